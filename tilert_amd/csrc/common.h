@@ -78,6 +78,39 @@ __device__ inline float group_scale(float amax, int scale_mode) {
   return amax * (1.0f / 448.0f);
 }
 
+// e4m3 codes of clamp(v / s, -448, 448) for 8 values of one group (s its scale), byte order =
+// value order.  Bit for bit the IEEE quotient followed by the RNE encode: the quotient comes from
+// r = RN(1 / s), once per group, with two fma residual corrections (Markstein: from a
+// faithful quotient and a correctly rounded reciprocal, one correction rounds
+// correctly; the first makes v * r faithful), 5 VALU operations where the division
+// expands to about 10, and v_cvt_pk_fp8_f32 encodes two values at a time (gfx950's fp8 is
+// e4m3fn, RNE) where f32_to_e4m3 takes about 12 operations each.  The residuals are exact
+// while s is far from the ends of the exponent range; other scales (and infinite ones)
+// divide.  A -0 quotient loses its sign in the residual sum, hence the copysign; a NaN
+// quotient becomes -448 in the clamp, on both paths.
+__device__ inline uint2 quant8_e4m3(const float (&v)[8], float s) {
+  float q[8];
+  if (s >= 0x1p-60f && s <= 0x1p60f) {
+    const float r = 1.0f / s;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float q0 = v[i] * r;
+      const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, s, v[i]), r, q0);
+      q[i] = __builtin_copysignf(__builtin_fmaf(__builtin_fmaf(-q1, s, v[i]), r, q1), v[i]);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) q[i] = v[i] / s;
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) q[i] = fminf(fmaxf(q[i], -kE4m3Max), kE4m3Max);
+  int lo = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], 0, false);
+  lo = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], lo, true);
+  int hi = __builtin_amdgcn_cvt_pk_fp8_f32(q[4], q[5], 0, false);
+  hi = __builtin_amdgcn_cvt_pk_fp8_f32(q[6], q[7], hi, true);
+  return make_uint2(static_cast<uint32_t>(lo), static_cast<uint32_t>(hi));
+}
+
 // ------------------------------------------------------------- wave reductions
 // OR of a 32-bit value over the wave's 64 lanes, wave-uniform.  An inclusive OR scan on
 // DPP (row shifts by 1, 2, 4, 8 within each 16-lane row, then the row broadcasts of lanes
