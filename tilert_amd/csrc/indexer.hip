@@ -415,17 +415,11 @@ __global__ __launch_bounds__(256) void ki_write_kernel(const uint16_t* __restric
   for (int i = 0; i < 8; ++i) amax = fmaxf(amax, __builtin_fabsf(v[i]));
   amax = row16_reduce<true>(amax);  // the group's 16 lanes
   const float sc = group_scale(amax, scale_mode);
-  uint32_t lo = 0, hi = 0;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    lo |= f32_to_e4m3(fminf(fmaxf(v[i] / sc, -kE4m3Max), kE4m3Max)) << (8 * i);
-    hi |= f32_to_e4m3(fminf(fmaxf(v[i + 4] / sc, -kE4m3Max), kE4m3Max)) << (8 * i);
-  }
   if (live) {
     const int64_t key = pos + row;
     uint8_t* page = pages + (key / kKiPageKeys) * kKiPageBytes;
     const int r = static_cast<int>(key % kKiPageKeys);
-    *reinterpret_cast<uint2*>(page + r * 128 + (tid & 15) * 8) = make_uint2(lo, hi);
+    *reinterpret_cast<uint2*>(page + r * 128 + (tid & 15) * 8) = quant8_e4m3(v, sc);
     if ((tid & 15) == 0) *reinterpret_cast<float*>(page + kKiPageKeys * 128 + r * 4) = sc;
   }
 }

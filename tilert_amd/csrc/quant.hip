@@ -27,14 +27,8 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const uint16_t* __restri
   for (int i = 0; i < 8; ++i) amax = fmaxf(amax, __builtin_fabsf(v[i]));
   amax = row16_reduce<true>(amax);  // the group's 16 lanes
   const float sc = group_scale(amax, scale_mode);
-  uint32_t lo = 0, hi = 0;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    lo |= f32_to_e4m3(fminf(fmaxf(v[i] / sc, -kE4m3Max), kE4m3Max)) << (8 * i);
-    hi |= f32_to_e4m3(fminf(fmaxf(v[i + 4] / sc, -kE4m3Max), kE4m3Max)) << (8 * i);
-  }
   if (live) {
-    reinterpret_cast<uint2*>(y)[tid] = make_uint2(lo, hi);
+    reinterpret_cast<uint2*>(y)[tid] = quant8_e4m3(v, sc);
     if ((tid & 15) == 0) s[grp] = sc;
   }
 }
@@ -228,7 +222,65 @@ constexpr int kNormPerThread = kNormVirt / kNormThreads;  // virtual threads per
 constexpr int kNormMaxChunks = 2;                           // chunks per virtual thread
 constexpr int kNormSlice = kNormThreads;                    // chunks per workgroup
 constexpr int kNormMaxDim = kNormMaxChunks * kNormVirt * 8;  // 16384
+constexpr int kNormRowsGrid = 1024;  // workgroups of the whole-row kernel (4 per CU; 512 and 2048 measured level)
+// Rows from which whole rows beat slices, by slices per row: a row of one slice (dim <= 2048) is a
+// whole row either way, without the sum's clamped loads (2.5 against 2.7 us at 1 row); up
+// to 8192 wide the redundant sums of the slices cost as much as the longer chain of a whole
+// row at 256 rows (dim 7168: 128 / 256 / 512 / 4096 rows 4.6 / 5.4 / 7.5 / 34.9 us against
+// 3.7 / 5.4 / 8.5 / 49.3; dim 3072: 3.4 / 3.6 / 4.5 / 17.3 against 3.1 / 3.6 / 5.0 / 21.4);
+// beyond that the registers of a whole row leave two workgroups per CU (dim 16384: 512 / 1024 /
+// 4096 rows 16.4 / 28.4 / 88 against 15.8 / 36.2 / 189).
+__host__ inline int64_t norm_rows_min(int64_t slices) { return slices <= 1 ? 1 : (slices <= 4 ? 256 : 1024); }
 
+__device__ inline float sum_squares(const uint4& raw, bool in, float ss) {
+  const uint32_t w4[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float lo = in ? bf16_to_f32(w4[j] & 0xffff) : 0.f;
+    const float hi = in ? bf16_to_f32(w4[j] >> 16) : 0.f;
+    ss = __builtin_fmaf(lo, lo, ss);
+    ss = __builtin_fmaf(hi, hi, ss);
+  }
+  return ss;
+}
+
+__device__ inline float norm_factor(const float (&part)[kNormVirt / 64], int dim, float eps) {
+  float tot = 0.f;
+#pragma unroll
+  for (int w = 0; w < kNormVirt / 64; ++w) tot += part[w];
+  return 1.0f / __builtin_sqrtf(tot / static_cast<float>(dim) + eps);
+}
+
+// Normalise (and quantise) chunk c of a row: 16 consecutive lanes hold a 128-element group.
+__device__ inline void norm_chunk(const uint4& raw, const float (&gv)[8], float r, bool live, int c, int row, int dim,
+                                  uint16_t* __restrict__ y, uint8_t* __restrict__ y8, float* __restrict__ ys,
+                                  int scale_mode) {
+  const uint32_t w4[4] = {raw.x, raw.y, raw.z, raw.w};
+  uint32_t b[4];  // bf16 pairs
+  float q[8];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const v2f f = {gv[2 * j] * (bf16_to_f32(w4[j] & 0xffff) * r), gv[2 * j + 1] * (bf16_to_f32(w4[j] >> 16) * r)};
+    b[j] = bf16x2_bits(f);
+    q[2 * j] = bf16_to_f32(b[j] & 0xffff);
+    q[2 * j + 1] = bf16_to_f32(b[j] >> 16);
+  }
+  if (live) reinterpret_cast<uint4*>(y + static_cast<int64_t>(row) * dim)[c] = make_uint4(b[0], b[1], b[2], b[3]);
+  if (!y8) return;  // kernel-uniform
+  float amax = 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) amax = fmaxf(amax, __builtin_fabsf(q[j]));
+  amax = row16_reduce<true>(amax);  // the group's 16 lanes
+  const float sc = group_scale(amax, scale_mode);
+  const uint2 code = quant8_e4m3(q, sc);
+  if (live) {
+    reinterpret_cast<uint2*>(y8 + static_cast<int64_t>(row) * dim)[c] = code;
+    if ((c & 15) == 0) ys[static_cast<int64_t>(row) * (dim / kBlock) + (c >> 4)] = sc;
+  }
+}
+
+// CH: chunks per virtual thread (1 up to dim 8192: no load or sum of chunks that are not there).
+template <int CH>
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_quant_kernel(
     const uint16_t* __restrict__ x, const float* __restrict__ gamma, float eps, int dim,
     uint16_t* __restrict__ y, uint8_t* __restrict__ y8, float* __restrict__ ys, int scale_mode) {
@@ -239,11 +291,11 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_quant_kernel(
   const bool live = c < nch;
   const uint4* xr = reinterpret_cast<const uint4*>(x + static_cast<int64_t>(row) * dim);
   // every load up front (clamped, unconditional): the row for the sum, this chunk, gamma
-  uint4 raw[kNormPerThread][kNormMaxChunks];
+  uint4 raw[kNormPerThread][CH];
 #pragma unroll
   for (int u = 0; u < kNormPerThread; ++u)
 #pragma unroll
-    for (int i = 0; i < kNormMaxChunks; ++i) raw[u][i] = xr[min(tid + u * kNormThreads + i * kNormVirt, nch - 1)];
+    for (int i = 0; i < CH; ++i) raw[u][i] = xr[min(tid + u * kNormThreads + i * kNormVirt, nch - 1)];
   const int cc = min(c, nch - 1);
   const uint4 mine = xr[cc];
   const float4 g0 = reinterpret_cast<const float4*>(gamma)[2 * cc];
@@ -252,55 +304,71 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_quant_kernel(
   for (int u = 0; u < kNormPerThread; ++u) {
     float ss = 0.f;
 #pragma unroll
-    for (int i = 0; i < kNormMaxChunks; ++i) {
-      const bool in = tid + u * kNormThreads + i * kNormVirt < nch;
-      const uint32_t w4[4] = {raw[u][i].x, raw[u][i].y, raw[u][i].z, raw[u][i].w};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float lo = in ? bf16_to_f32(w4[j] & 0xffff) : 0.f;
-        const float hi = in ? bf16_to_f32(w4[j] >> 16) : 0.f;
-        ss = __builtin_fmaf(lo, lo, ss);
-        ss = __builtin_fmaf(hi, hi, ss);
-      }
-    }
+    for (int i = 0; i < CH; ++i) ss = sum_squares(raw[u][i], tid + u * kNormThreads + i * kNormVirt < nch, ss);
     ss = wave_sum_f32(ss);
     if ((tid & 63) == 0) part[(tid >> 6) + u * (kNormThreads / 64)] = ss;
   }
   __syncthreads();
-  float tot = 0.f;
-#pragma unroll
-  for (int w = 0; w < kNormVirt / 64; ++w) tot += part[w];
-  const float r = 1.0f / __builtin_sqrtf(tot / static_cast<float>(dim) + eps);
+  const float r = norm_factor(part, dim, eps);
   const float gv[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-  const uint32_t w4[4] = {mine.x, mine.y, mine.z, mine.w};
-  uint16_t b[8];
-  float q[8];
+  norm_chunk(mine, gv, r, live, c, row, dim, y, y8, ys, scale_mode);
+}
+
+// Many rows (norm_rows_min): HBM-bound.  One workgroup takes whole rows, kept in registers between the sum and the outputs (the slices above read
+// and sum every row once per slice), strides over the rows with gamma held in registers -- as fp32
+// it is twice a row's bytes -- and requests its next row before it works on this one.  The sum is
+// the same tree: chunk tid + 256 j is virtual thread tid + 256 (j % 4)'s chunk j / 4.
+// 4096 x 7168 (147 MB moved): 34 us (4.3 TB/s) against 64 us for the slices, of which the
+// hardware conversions and the reciprocal quotient (quant8_e4m3) are 15 us.
+template <int NC>  // chunks per thread: dim <= 2048 NC
+__global__ __launch_bounds__(kNormThreads) void rmsnorm_quant_rows_kernel(
+    const uint16_t* __restrict__ x, const float* __restrict__ gamma, float eps, int rows, int dim,
+    uint16_t* __restrict__ y, uint8_t* __restrict__ y8, float* __restrict__ ys, int scale_mode) {
+  __shared__ float part[2][kNormVirt / 64];
+  const int tid = threadIdx.x, nch = dim / 8;
+  float gv[NC][8];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    b[2 * j] = f32_to_bf16(gv[2 * j] * (bf16_to_f32(w4[j] & 0xffff) * r));
-    b[2 * j + 1] = f32_to_bf16(gv[2 * j + 1] * (bf16_to_f32(w4[j] >> 16) * r));
+  for (int j = 0; j < NC; ++j) {
+    const int c = min(tid + j * kNormThreads, nch - 1);
+    const float4 g0 = reinterpret_cast<const float4*>(gamma)[2 * c], g1 = reinterpret_cast<const float4*>(gamma)[2 * c + 1];
+    gv[j][0] = g0.x; gv[j][1] = g0.y; gv[j][2] = g0.z; gv[j][3] = g0.w;
+    gv[j][4] = g1.x; gv[j][5] = g1.y; gv[j][6] = g1.z; gv[j][7] = g1.w;
   }
+  uint4 cur[NC], nxt[NC];
+  auto load = [&](int row, uint4 (&v)[NC]) {
+    const uint4* xr = reinterpret_cast<const uint4*>(x + static_cast<int64_t>(row) * dim);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) q[j] = bf16_to_f32(b[j]);
-  if (live)
-    reinterpret_cast<uint4*>(y + static_cast<int64_t>(row) * dim)[c] =
-        make_uint4(b[0] | (static_cast<uint32_t>(b[1]) << 16), b[2] | (static_cast<uint32_t>(b[3]) << 16),
-                   b[4] | (static_cast<uint32_t>(b[5]) << 16), b[6] | (static_cast<uint32_t>(b[7]) << 16));
-  if (!y8) return;  // kernel-uniform
-  float amax = 0.f;
+    for (int j = 0; j < NC; ++j) v[j] = xr[min(tid + j * kNormThreads, nch - 1)];
+  };
+  auto work = [&](int row, const uint4 (&v)[NC], float (&pt)[kNormVirt / 64]) {
 #pragma unroll
-  for (int j = 0; j < 8; ++j) amax = fmaxf(amax, __builtin_fabsf(q[j]));
-  amax = row16_reduce<true>(amax);  // the group's 16 lanes
-  const float sc = group_scale(amax, scale_mode);
-  uint32_t lo = 0, hi = 0;
+    for (int u = 0; u < kNormPerThread; ++u) {
+      float ss = 0.f;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    lo |= f32_to_e4m3(fminf(fmaxf(q[j] / sc, -kE4m3Max), kE4m3Max)) << (8 * j);
-    hi |= f32_to_e4m3(fminf(fmaxf(q[j + 4] / sc, -kE4m3Max), kE4m3Max)) << (8 * j);
-  }
-  if (live) {
-    reinterpret_cast<uint2*>(y8 + static_cast<int64_t>(row) * dim)[c] = make_uint2(lo, hi);
-    if ((c & 15) == 0) ys[static_cast<int64_t>(row) * (dim / kBlock) + (c >> 4)] = sc;
+      for (int j = u; j < NC; j += kNormPerThread)
+        ss = sum_squares(v[j], tid + j * kNormThreads < nch, ss);
+      ss = wave_sum_f32(ss);
+      if ((tid & 63) == 0) pt[(tid >> 6) + u * (kNormThreads / 64)] = ss;
+    }
+    __syncthreads();
+    const float r = norm_factor(pt, dim, eps);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const int c = tid + j * kNormThreads;
+      norm_chunk(v[j], gv[j], r, c < nch, c, row, dim, y, y8, ys, scale_mode);
+    }
+  };
+  // two rows a step, so that no row is copied between register sets; the partials alternate too:
+  // a row's are rewritten two rows later, after a barrier that follows every read of them
+  const int step = static_cast<int>(gridDim.x);
+  int row = blockIdx.x;
+  load(row, cur);
+  for (; row < rows; row += 2 * step) {
+    load(min(row + step, rows - 1), nxt);
+    work(row, cur, part[0]);
+    if (row + step >= rows) break;
+    load(min(row + 2 * step, rows - 1), cur);
+    work(row + step, nxt, part[1]);
   }
 }
 
@@ -328,9 +396,26 @@ extern "C" int tl_rmsnorm_quant(const void* x_bf16, const float* gamma, float ep
   if (rows == 0) return kOk;
   if (rows > 0x7fffffff) { set_error("rmsnorm_quant: too many rows (%lld)", (long long)rows); return kErrArg; }
   const unsigned slices = static_cast<unsigned>(cdiv(dim / 8, kNormSlice));
-  hipLaunchKernelGGL(rmsnorm_quant_kernel, dim3(static_cast<unsigned>(rows), slices), dim3(kNormThreads), 0,
-                     (hipStream_t)stream, (const uint16_t*)x_bf16, gamma, eps, (int)dim, (uint16_t*)y_bf16,
-                     (uint8_t*)y_fp8, y_scale, scale_mode);
+  if (rows < norm_rows_min(slices)) {
+    const dim3 grid(static_cast<unsigned>(rows), slices);
+    auto slice = [&](auto ch) {
+      hipLaunchKernelGGL((rmsnorm_quant_kernel<decltype(ch)::value>), grid, dim3(kNormThreads), 0, (hipStream_t)stream,
+                         (const uint16_t*)x_bf16, gamma, eps, (int)dim, (uint16_t*)y_bf16, (uint8_t*)y_fp8, y_scale, scale_mode);
+    };
+    if (dim <= kNormVirt * 8) slice(std::integral_constant<int, 1>{});
+    else slice(std::integral_constant<int, 2>{});
+    return check_launch("rmsnorm_quant");
+  }
+  auto launch = [&](auto nc) {
+    hipLaunchKernelGGL((rmsnorm_quant_rows_kernel<decltype(nc)::value>),
+                       dim3(static_cast<unsigned>(rows < kNormRowsGrid ? rows : kNormRowsGrid)), dim3(kNormThreads), 0,
+                       (hipStream_t)stream, (const uint16_t*)x_bf16, gamma, eps, (int)rows, (int)dim, (uint16_t*)y_bf16,
+                       (uint8_t*)y_fp8, y_scale, scale_mode);
+  };
+  if (slices <= 1) launch(std::integral_constant<int, 1>{});
+  else if (slices <= 2) launch(std::integral_constant<int, 2>{});
+  else if (slices <= 4) launch(std::integral_constant<int, 4>{});
+  else launch(std::integral_constant<int, 8>{});
   return check_launch("rmsnorm_quant");
 }
 
