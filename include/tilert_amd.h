@@ -92,9 +92,8 @@ int tl_weight_dequant(const void* q_fp8, const float* s, void* out, int out_bf16
 /* c[M,N] bf16 = (a . b^T) with per-128-K-block scaling, fp32 accumulation.
  * a fp8 [M,K], a_s fp32 [M,K/128], b fp8 [N,K], b_s fp32 [ceil(N/128),K/128].
  * Requires K % 128 == 0, N % 16 == 0, 1 <= M <= 256, 16-byte aligned a and b.
- * From M = 16 on (a rearranged copy of the activations, or the packed MFMA GEMM's split-K
- * partials from M = 17 or 33) and for narrow layers at M > 16 (split-K partials) the call needs
- * a workspace of tl_fp8_gemm_workspace_bytes(M,N,K)
+ * From M = 16 on (a rearranged copy of the activations, or the MFMA GEMM's counters and split-K
+ * partials) the call needs a workspace of tl_fp8_gemm_workspace_bytes(M,N,K)
  * bytes (0 = none), ZERO-FILLED before its first use; the kernels leave it ready for the
  * next call.  Calls that share a workspace must be ordered
  * (same stream).  Replaces fp8_gemm (refs/kernel.py:282-306). */
@@ -116,9 +115,8 @@ int tl_fp8_gemm(const void* a, const float* a_s, const void* b, const float* b_s
 int tl_fp8_pack_weight(const void* b, void* packed, int64_t N, int64_t K, void* stream);
 
 /* tl_fp8_gemm with b in the fragment-packed layout of tl_fp8_pack_weight (same scales,
- * same workspace rule).  Results equal tl_fp8_gemm's bit for bit where both run the GEMV
- * (M <= 16, or N % 128 != 0); from M = 17 or 33 with N % 128 == 0 the packed layout runs an MFMA
- * GEMM that sums the K blocks in another order (same tolerance against the reference).
+ * same workspace rule).  Results equal tl_fp8_gemm's bit for bit: both layouts run the same
+ * kernels in the same order of sums.
  * The FP8 GEMV / GEMM behind the reference's packed-weight projection ops (projx_wqkva_op,
  * rmsnorm_up_gate_silu_op, ...). */
 int tl_fp8_gemm_packed(const void* a, const float* a_s, const void* b_packed, const float* b_s,

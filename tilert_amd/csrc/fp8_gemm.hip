@@ -17,20 +17,14 @@
 //     each wave-wide load reads 1 KB of consecutive memory.  Packing is done once at
 //     weight-load time (tl_fp8_pack_weight), like the reference's per-op weight
 //     converters.  Measured on MI355X: packed fragments stream ~25% faster.
-//   * M <= 64 (fp8_gemm_kernel; on packed weights with N % 128 = 0 only up to M = 16, and
-//     at M = 17..32 where the wide kernel below would split K in more than 4): a workgroup
-//     owns one 16-row tile and a slice of K blocks;
-//     its 4-8 waves interleave over the slice, each with the next block's operands in
-//     flight (two buffers in ping-pong; deeper rings measured no faster), and are summed
-//     through LDS in a fixed order.  The K split is chosen so the grid covers the 256 CUs
-//     evenly; the last workgroup of a row tile (agent-scope counter and agent-scope atomic
-//     partials) sums the fp32 partials in slice order, so results are deterministic.
-//   * from M = 17 (K split in <= 4) or 33 on packed weights with N % 128 = 0
-//     (fp8_gemm_wide_kernel): F row
-//     tiles x 64 or 128 tokens per workgroup, one balanced round of 256 workgroups,
-//     operands staged in LDS.
-//   * M > 64 otherwise (fp8_gemm_tiled_kernel): 128-row workgroups share activation chunks
-//     staged in LDS (see below).
+//   * M <= 16, and some layers up to M = 32 (fp8_gemm_kernel): a workgroup
+//     owns one or two 16-row tiles over the whole K; its 4 or 8 waves interleave over the
+//     K blocks, each with the next block's operands in flight (two buffers in ping-pong;
+//     deeper rings measured no faster on narrow layers), and are summed through LDS in a
+//     fixed order.
+//   * larger M (fp8_gemm_wide_kernel): F row tiles x 64 or 128 tokens per workgroup, one
+//     round of at most 256 workgroups, operands staged in LDS.
+// Both take either weight layout with the same plan, so the layouts' results are equal bit for bit.
 #include <algorithm>
 #include <cstdint>
 #include <type_traits>
@@ -122,10 +116,8 @@ __device__ inline void store_out(const OutRoute& o, int t, int n, uint2 v) {
   *reinterpret_cast<uint2*>(dst) = v;
 }
 
-// D: operand buffers per wave.  D = 2 is the ping-pong below; narrow layers (few row
-// tiles, so few waves on the chip) take a deeper ring so that enough weight bytes are in
-// flight to cover HBM latency without splitting K.
-// RT: 16-row tiles per workgroup (1, 2 or 4; within one 128-row scale block).  Each
+// D: operand buffers per wave (2: the ping-pong below; 4 on wide, long layers).
+// RT: 16-row tiles per workgroup (1 or 2; within one 128-row scale block).  Each
 // activation fragment a wave loads then serves RT weight fragments, which divides the
 // activation traffic (as large as the weight traffic itself from M = 16 on) by RT.
 // XF: A / As are the activation image of act_image_kernel (fragment order, transposed
@@ -133,16 +125,11 @@ __device__ inline void store_out(const OutRoute& o, int t, int n, uint2 v) {
 template <int MT, int WAVES, bool PACKED, int D = 2, int RT = 1, bool XF = false>
 __global__ __launch_bounds__(WAVES * 64) void fp8_gemm_kernel(
     const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ B,
-    const float* __restrict__ Bs, const OutRoute out, float* __restrict__ partial,
-    uint32_t* __restrict__ counters, int M, int N, int K, int kb_per_split) {
+    const float* __restrict__ Bs, const OutRoute out, int M, int N, int K) {
   constexpr int NA = RT * MT;  // accumulators per lane: (row tile j, token tile mt) at j * MT + mt
   __shared__ v4f red[WAVES - 1][NA][64];
   const int KB = K >> 7;
   const int NT = N >> 4;
-  const int ksplit = gridDim.y;
-  const int ks = blockIdx.y;
-  const int kb_begin = ks * kb_per_split;
-  const int kb_end = min(KB, kb_begin + kb_per_split);
   const int rt = blockIdx.x * RT;  // first row tile
   const int n0 = rt * 16;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -197,9 +184,9 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_gemm_kernel(
       for (int j = 0; j < RT; ++j) acc[j * MT + mt] += mfma_16x16x128_fp8(o.a[j], o.x[mt]) * (o.bs * xs);
     }
   };
-  // this wave's K blocks: kb_begin + wv + i*WAVES, i < n
-  const int kb0 = kb_begin + wv;
-  const int n = kb0 < kb_end ? (kb_end - kb0 + WAVES - 1) / WAVES : 0;
+  // this wave's K blocks: wv + i*WAVES, i < n
+  const int kb0 = wv;
+  const int n = kb0 < KB ? (KB - kb0 + WAVES - 1) / WAVES : 0;
   if constexpr (D > 2) {
     Ops ring[D];
     ring_pipeline<D>(n, ring, [&](int i, Ops& o) { fetch(kb0 + i * WAVES, o); },
@@ -238,57 +225,11 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_gemm_kernel(
     for (int i = 0; i < NA; ++i) acc[i] += red[w][i][lane];
 
   // lane holds output columns n0 + 16 jt + 4g + j (j = 0..3) of token mt*16 + r
-  if (ksplit == 1) {
-#pragma unroll
-    for (int i = 0; i < NA; ++i) {
-      const int t = (i % MT) * 16 + r;
-      if (t < M) store_out(out, t, n0 + 16 * (i / MT) + 4 * g, pack_bf16x4(acc[i]));
-    }
-    return;
-  }
-
-  // ---- split-K: publish fp32 partials; the last slice to arrive reduces them in order.
-  // Partials are agent-scope atomic stores/loads (written through to the device
-  // coherence point, read past this XCD's L2), so no cache-wide writeback or
-  // invalidate is needed; s_waitcnt makes the stores complete before the counter bump.
 #pragma unroll
   for (int i = 0; i < NA; ++i) {
     const int t = (i % MT) * 16 + r;
-    if (t < M) {
-      float* dst = partial + (static_cast<size_t>(ks) * M + t) * N + n0 + 16 * (i / MT) + 4 * g;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) __hip_atomic_store(dst + j, acc[i][j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (t < M) store_out(out, t, n0 + 16 * (i / MT) + 4 * g, pack_bf16x4(acc[i]));
   }
-  __builtin_amdgcn_s_waitcnt(0);
-  uint32_t prev = 0;
-  if (lane == 0) prev = __hip_atomic_fetch_add(&counters[rt], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  prev = __shfl(prev, 0);
-  if (prev != static_cast<uint32_t>(ksplit - 1)) return;
-#pragma unroll
-  for (int i = 0; i < NA; ++i) {
-    const int t = (i % MT) * 16 + r;
-    const int ncol = n0 + 16 * (i / MT) + 4 * g;
-    if (t < M) {
-      // issue the loads of 8 slices at a time, then add them in slice order
-      v4f s = {0.f, 0.f, 0.f, 0.f};
-      for (int q0 = 0; q0 < ksplit; q0 += 8) {
-        v4f v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const int q = q0 + u < ksplit ? q0 + u : ksplit - 1;
-          const float* src = partial + (static_cast<size_t>(q) * M + t) * N + ncol;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) v[u][j] = __hip_atomic_load(src + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-          if (q0 + u < ksplit) s += v[u];
-      }
-      store_out(out, t, ncol, pack_bf16x4(s));
-    }
-  }
-  if (lane == 0) __hip_atomic_store(&counters[rt], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Pack a canonical [N, K] fp8 weight into K-group-major MFMA fragments (see
@@ -311,7 +252,7 @@ __global__ __launch_bounds__(256) void pack_weight_kernel(const uint8_t* __restr
       *reinterpret_cast<const uint4*>(W + static_cast<size_t>(row) * K + col);
 }
 
-// Activation image for the GEMVs at M > 16: x [M, K] rearranged so that the MFMA operand
+// Activation image for the GEMVs at M >= 16: x [M, K] rearranged so that the MFMA operand
 // of token tile tt and K block kb is 2 KB of consecutive memory at (kb * MTT + tt) * 2048
 // (MTT = ceil(M / 16); in-fragment order as in the weight packing; tokens past M repeat
 // token M-1), and the scales transposed to [K/128, 16 MTT] (0 past M).  The GEMV's
@@ -359,20 +300,6 @@ __global__ __launch_bounds__(256) void pack_tile_major_kernel(const uint8_t* __r
   reinterpret_cast<uint4*>(P)[chunk] = *reinterpret_cast<const uint4*>(W + static_cast<size_t>(row) * K + col);
 }
 
-// ---------------------------------------------------------------- M > 64: tiled
-// For M > 64 tokens the activation blocks are no longer small next to the weights: a
-// wave that reads them from L1/L2 for each of its token tiles moves up to 4x the weight
-// bytes through the texture path.  Here a workgroup of 8 waves covers 128 rows (one
-// 16-row tile per wave) x all TT token tiles over a slice of K blocks:
-//   * activations (MFMA fragment order) and their scales are staged in LDS by the whole
-//     workgroup in chunks of KC = 16 / TT K blocks (32 KB), double-buffered and loaded
-//     one chunk ahead -- one barrier per chunk;
-//   * each wave streams its weight fragments through a ring of kTiledDepth buffers that
-//     runs on across chunk boundaries, so a barrier never drains the weight stream;
-//   * full chunks issue unconditional loads only (exact wait counts); the last chunks of
-//     a slice guard the weight fetches, so no fragment is read twice.
-// Split-K slices are reduced as in fp8_gemm_kernel (partials + last-arriver, in slice
-// order, deterministic).
 // static_for<N>(f): f(std::integral_constant<int, 0>{}) ... f(<N-1>) -- compile-time loop
 template <int... I, class F>
 __device__ __attribute__((always_inline)) inline void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
@@ -383,216 +310,8 @@ __device__ __attribute__((always_inline)) inline void static_for(F&& f) {
   static_for_impl(std::make_integer_sequence<int, N>{}, f);
 }
 
-constexpr int kTiledWaves = 8;
-constexpr int kTiledDepth = 4;
-
-template <int TT>
-struct TiledShape {
-  static constexpr int THREADS = kTiledWaves * 64;
-  static constexpr int KC = 16 / TT >= 1 ? 16 / TT : 1;   // K blocks per chunk
-  static_assert(KC % kTiledDepth == 0 || kTiledDepth % KC == 0, "ring slots must be static");
-  static constexpr int XCH = KC * TT * 128;                // 16-byte chunks per chunk
-  static constexpr int XPT = (XCH + THREADS - 1) / THREADS;
-  static constexpr int XBUF = XPT * THREADS * 16;          // bytes per buffer (padded)
-  static constexpr int SCN = KC * TT * 16;                 // activation scales per chunk
-  static constexpr int SPT = (SCN + THREADS - 1) / THREADS;
-  static constexpr int SBUF = SPT * THREADS;               // floats per buffer (padded)
-  static constexpr int LDS = 2 * XBUF + 2 * SBUF * 4;
-};
-
-// dynamic LDS of fp8_gemm_tiled_kernel<TT>
-template <int TT>
-constexpr int tiled_lds_bytes() { return TiledShape<TT>::LDS; }
-
-template <int TT, bool PACKED>
-__global__ __launch_bounds__(kTiledWaves * 64) void fp8_gemm_tiled_kernel(
-    const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ B,
-    const float* __restrict__ Bs, const OutRoute out, float* __restrict__ partial,
-    uint32_t* __restrict__ counters, int M, int N, int K, int kb_per_split) {
-  using S = TiledShape<TT>;
-  constexpr int KC = S::KC, D = kTiledDepth, THREADS = S::THREADS;
-  extern __shared__ __attribute__((aligned(16))) uint8_t tiled_smem[];
-  __shared__ uint32_t last_flag;
-  const int KB = K >> 7;
-  const int NT = N >> 4;
-  const int ksplit = gridDim.y, ks = blockIdx.y;
-  const int kb_begin = ks * kb_per_split;
-  const int n = max(0, min(KB, kb_begin + kb_per_split) - kb_begin);  // K blocks in this slice
-  const int nch = (n + KC - 1) / KC;                                  // chunks
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r = lane & 15, g = lane >> 4;
-  const int rt = min(static_cast<int>(blockIdx.x) * kTiledWaves + wave, NT - 1);  // rows past N: not stored
-  const bool row_ok = static_cast<int>(blockIdx.x) * kTiledWaves + wave < NT;
-  const uint8_t* brow = B + static_cast<size_t>(rt * 16 + r) * K;
-  const float* bs_row = Bs + static_cast<size_t>(rt >> 3) * KB;
-
-  // ---- activation chunks: chunk c covers K blocks kb_begin + c*KC + j, j < KC.  LDS
-  // image chunk d: block j = d / (TT*128), token tile tt = (d / 128) % TT, piece
-  // (d / 64) % 2, lane d % 64 -> token 16 tt + l % 16 (clamped), 16-byte piece 4 p + l / 16
-  u32x4 xr[S::XPT];  // ext-vector type: a HIP uint4 struct copy would stay in scratch
-  float sr[S::SPT];
-  auto x_issue = [&](int c) __attribute__((always_inline)) {  // unconditional, indices clamped
-    static_for<S::XPT>([&](auto ut) __attribute__((always_inline)) {
-      constexpr int u = decltype(ut)::value;
-      const int d = min(tid + u * THREADS, S::XCH - 1);
-      const int j = d / (TT * 128), tt = (d >> 7) % TT, pp = (d >> 6) & 1, l = d & 63;
-      const int kb = kb_begin + min(c * KC + j, n - 1);
-      const int tok = min(tt * 16 + (l & 15), M - 1);
-      xr[u] = *reinterpret_cast<const u32x4*>(A + static_cast<size_t>(tok) * K + kb * kBlock + pp * 64 + (l >> 4) * 16);
-    });
-    static_for<S::SPT>([&](auto ut) __attribute__((always_inline)) {
-      constexpr int u = decltype(ut)::value;
-      const int e = min(tid + u * THREADS, S::SCN - 1);  // scale e: block e / (TT*16), token e % (TT*16)
-      const int kb = kb_begin + min(c * KC + e / (TT * 16), n - 1);
-      sr[u] = As[static_cast<size_t>(min(e % (TT * 16), M - 1)) * KB + kb];
-    });
-  };
-  auto x_put = [&](int buf) __attribute__((always_inline)) {  // unconditional writes (padding absorbs the surplus)
-    u32x4* xl = reinterpret_cast<u32x4*>(tiled_smem + buf * S::XBUF);
-    float* sl = reinterpret_cast<float*>(tiled_smem + 2 * S::XBUF) + buf * S::SBUF;
-    static_for<S::XPT>([&](auto ut) __attribute__((always_inline)) { xl[tid + decltype(ut)::value * THREADS] = xr[decltype(ut)::value]; });
-    static_for<S::SPT>([&](auto ut) __attribute__((always_inline)) {
-      constexpr int u = decltype(ut)::value;
-      const int e = tid + u * THREADS;
-      sl[e] = (e % (TT * 16)) < M ? sr[u] : 0.f;  // tokens past M contribute 0
-    });
-  };
-
-  // ---- weight ring: item i = K block kb_begin + i
-  v8i wr[D];
-  float bsr[D];
-  // slot = i % D, always passed as a compile-time value (a runtime index would put the
-  // ring in scratch memory)
-  auto w_fetch = [&](int i, auto slot_tag) __attribute__((always_inline)) {
-    constexpr int slot = decltype(slot_tag)::value;
-    const int kb = kb_begin + min(i, n - 1);
-    wr[slot] = PACKED ? load_packed_fragment(B + packed_fragment(rt, kb, NT), lane)
-                      : load_kblock_stream(brow + static_cast<size_t>(kb) * kBlock, g);
-    bsr[slot] = bs_row[kb];
-  };
-
-  v4f acc[TT];
-#pragma unroll
-  for (int tt = 0; tt < TT; ++tt) acc[tt] = v4f{0.f, 0.f, 0.f, 0.f};
-  auto compute = [&](auto slot_tag, int buf, int j) __attribute__((always_inline)) {  // chunk block j of buffer buf
-    constexpr int slot = decltype(slot_tag)::value;
-    const u32x4* xl = reinterpret_cast<const u32x4*>(tiled_smem + buf * S::XBUF) + j * TT * 128;
-    const float* sl = reinterpret_cast<const float*>(tiled_smem + 2 * S::XBUF) + buf * S::SBUF + j * TT * 16;
-#pragma unroll
-    for (int tt = 0; tt < TT; ++tt) {
-      const u32x4 lo = xl[tt * 128 + lane];
-      const u32x4 hi = xl[tt * 128 + 64 + lane];
-      const v8i xb = {static_cast<int>(lo.x), static_cast<int>(lo.y), static_cast<int>(lo.z), static_cast<int>(lo.w),
-                      static_cast<int>(hi.x), static_cast<int>(hi.y), static_cast<int>(hi.z), static_cast<int>(hi.w)};
-      acc[tt] += mfma_16x16x128_fp8(wr[slot], xb) * (bsr[slot] * sl[tt * 16 + r]);
-      if ((tt & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // bound the operand reads in flight
-    }
-  };
-
-  if (n > 0) {
-    // prologue: chunk 0 into LDS buffer 0, chunk 1 into registers, the first D-1 weights
-    x_issue(0);
-    x_put(0);
-    x_issue(1);
-    static_for<D - 1>([&](auto i) __attribute__((always_inline)) { w_fetch(decltype(i)::value, i); });
-    // one chunk: stage chunk c+1 (registers -> LDS), request chunk c+2, then its KC
-    // items.  CC = c % CPI is compile-time, so every ring slot is.  SAFE: every weight
-    // fetch of the chunk is inside the slice (no guard needed).
-    auto chunk = [&](int c, auto cc_tag, auto safe_tag) __attribute__((always_inline)) {
-      constexpr int CC = decltype(cc_tag)::value;
-      constexpr bool SAFE = decltype(safe_tag)::value;
-      __syncthreads();   // chunk c-1 is done everywhere: its buffer may be refilled
-      x_put((c + 1) & 1);
-      x_issue(c + 2);
-      static_for<KC>([&](auto jt) __attribute__((always_inline)) {
-        constexpr int j = decltype(jt)::value;
-        const int i = c * KC + j;
-        const auto cur = std::integral_constant<int, (CC * KC + j) % D>{};
-        const auto nxt = std::integral_constant<int, (CC * KC + j + D - 1) % D>{};
-        if (SAFE) {
-          w_fetch(i + D - 1, nxt);
-          compute(cur, c & 1, j);
-        } else if (i < n) {
-          if (i + D - 1 < n) w_fetch(i + D - 1, nxt);
-          compute(cur, c & 1, j);
-        }
-      });
-    };
-    __syncthreads();  // chunk 0 visible
-    // CPI chunks per loop step, unrolled, so that item i's ring slot i % D is a
-    // compile-time index (CPI * KC is a multiple of D)
-    constexpr int CPI = KC >= D ? 1 : D / KC;
-    int c = 0;
-    // a step is safe when its last fetch, item (c+CPI)*KC + D - 2, is inside the slice
-    for (; (c + CPI) * KC + D - 2 < n; c += CPI)
-      static_for<CPI>([&](auto cc) __attribute__((always_inline)) { chunk(c + decltype(cc)::value, cc, std::true_type{}); });
-    for (; c < nch; c += CPI)
-      static_for<CPI>([&](auto cc) __attribute__((always_inline)) {
-        if (c + decltype(cc)::value < nch) chunk(c + decltype(cc)::value, cc, std::false_type{});
-      });
-  }
-
-  // lane holds output rows rt*16 + 4g + j (j = 0..3) of token tt*16 + r
-  const int ncol = rt * 16 + 4 * g;
-  if (ksplit == 1) {
-    if (row_ok) {
-#pragma unroll
-      for (int tt = 0; tt < TT; ++tt) {
-        const int t = tt * 16 + r;
-        if (t < M) store_out(out, t, ncol, pack_bf16x4(acc[tt]));
-      }
-    }
-    return;
-  }
-  // split-K: agent-scope partials, then the last slice of this row group sums them
-  if (row_ok) {
-#pragma unroll
-    for (int tt = 0; tt < TT; ++tt) {
-      const int t = tt * 16 + r;
-      if (t < M) {
-        float* dst = partial + (static_cast<size_t>(ks) * M + t) * N + ncol;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) __hip_atomic_store(dst + j, acc[tt][j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-    }
-  }
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();  // every wave's partials are complete before the counter moves
-  if (tid == 0) {
-    const uint32_t prev = __hip_atomic_fetch_add(&counters[blockIdx.x], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    last_flag = prev == static_cast<uint32_t>(ksplit - 1);
-  }
-  __syncthreads();
-  if (!last_flag) return;
-  if (row_ok) {
-#pragma unroll
-    for (int tt = 0; tt < TT; ++tt) {
-      const int t = tt * 16 + r;
-      if (t < M) {
-        v4f s = {0.f, 0.f, 0.f, 0.f};
-        for (int q0 = 0; q0 < ksplit; q0 += 8) {
-          v4f v[8];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) {
-            const int q = q0 + u < ksplit ? q0 + u : ksplit - 1;
-            const float* src = partial + (static_cast<size_t>(q) * M + t) * N + ncol;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) v[u][j] = __hip_atomic_load(src + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          }
-#pragma unroll
-          for (int u = 0; u < 8; ++u)
-            if (q0 + u < ksplit) s += v[u];
-        }
-        store_out(out, t, ncol, pack_bf16x4(s));
-      }
-    }
-  }
-  if (tid == 0) __hip_atomic_store(&counters[blockIdx.x], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// ---------------------------------------------------------------- M > 32: MFMA GEMM
-// Wide-tile MFMA GEMM for 16 < M <= 256 on packed weights (fp8_gemm_wide_kernel<F, TJ>).
+// ---------------------------------------------------------------- M > 16: MFMA GEMM
+// Wide-tile MFMA GEMM for 16 < M <= 256 (fp8_gemm_wide_kernel<F, TJ, PACKED>).
 // A workgroup (8 waves, one workgroup per CU) owns F consecutive 16-row weight tiles x one
 // group of 4 TJ token fragments (64 or 128 tokens; TJ = 1 up to M = 64) over one of S K
 // ranges.  The host picks F (4..9) and S so that tiles x token groups x S <= 256
@@ -617,16 +336,18 @@ __global__ __launch_bounds__(kTiledWaves * 64) void fp8_gemm_tiled_kernel(
 // read with 16-byte sc1 accesses (past this XCD's L2, like agent-scope atomics); the
 // workgroup that completes a tile (agent-scope counter) sums them in range order, so
 // results are deterministic.
-// When the wide kernel replaces the GEMV on packed weights (measured, us, wide vs GEMV):
-// from M = 33 on always (up 7168 -> 18432 at M = 33 / 48 / 64: 28.1 / 28.7 / 29.5 vs
-// 48.9 / 49.1 / 51.2; down 18432 -> 7168 at M = 64: 29.8 vs 41.3; 7168 -> 1536 at M = 64:
-// 12.7 vs 22.5); at M = 17..32 only when its plan splits K at most in 4 (up at M = 17 / 32:
-// 28.5 / 27.9 vs 35.7 / 35.8; down at M = 17 / 24 / 32: 29.4 / 29.1 / 29.4 vs 30.2 / 30.3 /
-// 30.3; small layers that split K 8 ways or more lose: 7168 -> 1024 at M = 32 14.3 vs
-// 10.5, 2048 -> 4096 at M = 24 9.5 vs 6.5); at M <= 16 never (up at M = 16: GEMV 27.2).
-constexpr int kWideMinM = 32;      // from M = 33 on always
-constexpr int kWideMinM2 = 16;     // from M = 17 on when the K split is small:
-constexpr int kWideMaxSplit2 = 4;  // at most this many K ranges
+// Against the GEMV (us, wide / GEMV, packed): from M = 33 on always (7168 -> 18432 / 1536 /
+// 576 at M = 64: 29.8 / 49.8, 11.7 / 22.9, 10.3 / 15.0; 512 -> 4096 5.0 / 5.9; 1536 -> 3072
+// level); at M = 17..32 but for layers whose 16-row tiles give the GEMV one workgroup on
+// 192..256 CUs with no K split and a short stream (1536 -> 3072 at M = 24: 7.7 / 6.2;
+// 2048 -> 4096 9.6 / 6.8; 4096 -> 4096 11.0 / 9.1; next to them 2048 -> 2048 8.3 / 9.3 and
+// 4096 -> 5120 10.5 / 12.3; 512 -> 4096 4.9 / 5.3); at M <= 16 never (7168 -> 18432 at M = 16
+// 28.3 / 26.9, 7168 -> 1536 11.8 / 8.3).
+constexpr int kWideMinM = 32;   // from M = 33 on always
+constexpr int kWideMinM2 = 16;  // from M = 17 on but for
+constexpr int kGemvTiles0 = 192, kGemvTiles1 = 256;  // 16-row tiles and
+constexpr int kGemvKb0 = 8, kGemvKb1 = 32;           // K blocks in these ranges
+constexpr int kWideMaxSplit = 32;  // K ranges
 constexpr int kWideGrid = 256;
 constexpr int kCpolSc1 = 16;            // buffer access cache policy: sc1
 constexpr int kRsrcWord3 = 0x00020000;  // buffer resource word 3: 32-bit data format
@@ -640,12 +361,14 @@ constexpr int kWideWaves = 8;
 template <int F, int TJ>
 struct WideShape {
   static constexpr int TT = 4 * TJ;
-  static constexpr int STAGES = 4;                      // ring depth (5 measured no faster at TJ = 1)
   static constexpr int FH = (F + 1) / 2;                // rows of the first split
   static constexpr int W = F * 2048;                    // weight fragments of one K block
   static constexpr int A = TT * 2048;                   // activation fragments
   static constexpr int WS = W + A;                      // weight scales (F floats)
   static constexpr int STAGE = WS + 256;
+  // Ring depth.  Deeper rings measured no faster, also for layers of few workgroups: a block's
+  // copies take the CU's address unit about 0.02 us each, which no lead hides.
+  static constexpr int STAGES = 4;
   static constexpr int WIN = STAGES * STAGE;            // token-scale windows: [2][128][16] fp32
   static constexpr int LDS = WIN + 2 * 128 * 16 * 4;
   static constexpr int SLOT = F * TT * 256;             // floats of one partial
@@ -676,7 +399,7 @@ __device__ inline void dma_lds4(const void* src, uint32_t lds) {
                : "=&s"(saved) : "v"(src), "s"(__builtin_amdgcn_readfirstlane(lds)) : "memory");
 }
 
-template <int F, int TJ>
+template <int F, int TJ, bool PACKED>
 __global__ __launch_bounds__(kWideWaves * 64) void fp8_gemm_wide_kernel(
     const uint8_t* __restrict__ X, const float* __restrict__ Xs, const uint8_t* __restrict__ B,
     const float* __restrict__ Bs, const OutRoute out, float* __restrict__ partial,
@@ -690,7 +413,7 @@ __global__ __launch_bounds__(kWideWaves * 64) void fp8_gemm_wide_kernel(
   // id -> (weight slice q, token group tg): the groups of one slice are 8 ids apart
   const int id = static_cast<int>(blockIdx.x);
   const int q = (id / (8 * TG)) * 8 + id % 8, tg = (id / 8) % TG;
-  if (q >= (NT / F) * S) return;  // padding ids of the last group of 8 slices
+  if (q >= (NT + F - 1) / F * S) return;  // padding ids of the last group of 8 slices
   const int tile = q / S, seg = q % S;
   const int kb0 = seg * per;
   const int n = KB - kb0 < per ? KB - kb0 : per;  // >= 1 (host plan)
@@ -721,7 +444,9 @@ __global__ __launch_bounds__(kWideWaves * 64) void fp8_gemm_wide_kernel(
                        min(t0 + 16 * wave + 8 + (lane >> 4), M - 1), min(t0 + 16 * wave + 12 + (lane >> 4), M - 1)};
   const int sblk = lane & 15;
   const int fr = lane < F - 1 ? lane : F - 1;
-  const float* ws_src = Bs + static_cast<size_t>((16 * (F * tile + fr)) >> 7) * KB;  // weight scales (wave 2)
+  // weight scales (wave 2); row fragments past the weight's last one (NT not a multiple of F)
+  // repeat it, here and in the pieces below, and are not stored
+  const float* ws_src = Bs + static_cast<size_t>((16 * min(F * tile + fr, NT - 1)) >> 7) * KB;
 
   // this lane's weight pieces at K block 0 (a block's fragments lie a fixed offset further)
   constexpr int WPW = (2 * F + kWideWaves - 1) / kWideWaves;
@@ -729,7 +454,11 @@ __global__ __launch_bounds__(kWideWaves * 64) void fp8_gemm_wide_kernel(
 #pragma unroll
   for (int u = 0; u < WPW; ++u) {
     const int p = wave + kWideWaves * u < 2 * F - 1 ? wave + kWideWaves * u : 2 * F - 1;
-    wsrc[u] = B + packed_fragment(F * tile + (p >> 1), 0, NT) + (p & 1) * 1024 + lane * 16;
+    const int t = min(F * tile + (p >> 1), NT - 1);
+    // packed: half a fragment, 1 KB of consecutive memory; stored [N, K]: 8 rows' 128 bytes,
+    // swizzled as the activations are
+    wsrc[u] = PACKED ? B + packed_fragment(t, 0, NT) + (p & 1) * 1024 + lane * 16
+                     : B + static_cast<size_t>(16 * t + 8 * (p & 1) + (lane >> 3)) * K + achunk * 16;
   }
   const uint32_t lds0 =
       __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_u8_ptr)smem)));
@@ -737,7 +466,7 @@ __global__ __launch_bounds__(kWideWaves * 64) void fp8_gemm_wide_kernel(
   // copies of K block kb into stage sidx
   auto issue = [&](int kb, int sidx) {
     const uint32_t ls = lds0 + sidx * Sh::STAGE;
-    const size_t koff = (static_cast<size_t>(kb >> 2) * NT * kGroup + (kb & 3)) * 2048;
+    const size_t koff = PACKED ? (static_cast<size_t>(kb >> 2) * NT * kGroup + (kb & 3)) * 2048 : static_cast<size_t>(kb) * kBlock;
 #pragma unroll
     for (int u = 0; u < WPW; ++u) {
       const int p = wave + kWideWaves * u;  // fragment p / 2, half p % 2
@@ -781,15 +510,14 @@ __global__ __launch_bounds__(kWideWaves * 64) void fp8_gemm_wide_kernel(
       v8i a[TJ], w[NR];
       float ts[TJ], ws[NR];
     };
-    auto stage = [&](int i) { return smem + (i % Sh::STAGES) * Sh::STAGE; };
     auto last = [&](int i) { return kb0 + (i < n - 1 ? i : n - 1); };  // past the range: re-copy the last block
-    auto load = [&](int i, Ops& o) {  // block kb0 + i (past the range: unused values)
-      const uint8_t* st = stage(i);
+    auto load = [&](int i, int sidx, Ops& o) {  // block kb0 + i from its stage (past the range: unused values)
+      const uint8_t* st = smem + sidx * Sh::STAGE;
       const int kb = kb0 + i;
 #pragma unroll
       for (int j = 0; j < TJ; ++j) o.a[j] = load_act(st + Sh::W + (TJ * tp + j) * 2048);
 #pragma unroll
-      for (int f = 0; f < NR; ++f) o.w[f] = load_fragment(st + (f0 + f) * 2048, lane);
+      for (int f = 0; f < NR; ++f) o.w[f] = PACKED ? load_fragment(st + (f0 + f) * 2048, lane) : load_act(st + (f0 + f) * 2048);
       const float* tsr = reinterpret_cast<const float*>(smem + Sh::WIN + ((kb >> 4) & 1) * 8192) +
                          (16 * TJ * tp + r) * 16 + (kb & 15);
       const float* wsr = reinterpret_cast<const float*>(st + Sh::WS) + f0;
@@ -821,13 +549,16 @@ __global__ __launch_bounds__(kWideWaves * 64) void fp8_gemm_wide_kernel(
     __builtin_amdgcn_s_waitcnt(vmcnt_imm((SN - 2) * OPS));  // block 0 landed
     asm volatile("s_barrier" ::: "memory");
     Ops o0, o1;
-    load(0, o0);
+    load(0, 0, o0);
+    int rd = 1, wr = SN - 1;  // stages of block i + 1 and of block i + SN - 1
     auto step = [&](int i, const Ops& cur, Ops& nxt) {
       __builtin_amdgcn_s_waitcnt(vmcnt_imm((SN - 3) * OPS));  // block i + 1 landed (not i + 2 .. i + SN - 2)
       asm volatile("s_barrier" ::: "memory");
-      issue(last(i + SN - 1), (i + SN - 1) % SN);
-      load(i + 1, nxt);  // unconditional (past the range it reads a stage unused): no
-      mma(cur);          // branch, so the wait for cur's reads stays partial
+      issue(last(i + SN - 1), wr);
+      load(i + 1, rd, nxt);  // unconditional (past the range it reads a stage unused): no
+      mma(cur);              // branch, so the wait for cur's reads stays partial
+      rd = rd + 1 < SN ? rd + 1 : 0;
+      wr = wr + 1 < SN ? wr + 1 : 0;
     };
     for (int i = 0; i < n; i += 2) {
       step(i, o0, o1);
@@ -843,8 +574,15 @@ __global__ __launch_bounds__(kWideWaves * 64) void fp8_gemm_wide_kernel(
     else if (ops == OPS_LO + 1) run(nr_tag, std::integral_constant<int, OPS_LO + 1>{});
     else run(nr_tag, std::integral_constant<int, OPS_LO + 2>{});
   };
-  if (rh == 0) by_ops(std::integral_constant<int, FH>{});
-  else by_ops(std::integral_constant<int, F - FH>{});
+  // (F even: one call site.  Called twice with the same type, the body becomes a function of its own
+  // that takes every captured value, register sets included, through scratch memory: F = 4, 6 and
+  // 8 ran 3 to 4 times slower than their neighbours)
+  if constexpr (2 * FH == F) {
+    by_ops(std::integral_constant<int, FH>{});
+  } else {
+    if (rh == 0) by_ops(std::integral_constant<int, FH>{});
+    else by_ops(std::integral_constant<int, F - FH>{});
+  }
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // no copy may land after the workgroup ends
 
   // lane holds rows 16 (F tile + f0 + f) + 4 g + (0..3) of token 16 (tf0 + j) + r
@@ -856,7 +594,7 @@ __global__ __launch_bounds__(kWideWaves * 64) void fp8_gemm_wide_kernel(
     for (int f = 0; f < FH; ++f)
 #pragma unroll
       for (int j = 0; j < TJ; ++j)
-        if (f < nrows && token(j) < M) store_out(out, token(j), column(f), pack_bf16x4(acc[f][j]));
+        if (f < nrows && token(j) < M && column(f) < N) store_out(out, token(j), column(f), pack_bf16x4(acc[f][j]));
   };
   if (S == 1) {
     store_all();
@@ -902,31 +640,57 @@ __global__ __launch_bounds__(kWideWaves * 64) void fp8_gemm_wide_kernel(
   if (tid == 0) __hip_atomic_store(&counters[tile * TG + tg], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Plan of the wide kernel: F (row tiles per workgroup, 4..9, dividing N / 16) and the K
-// split S minimising rounds x F x (K blocks per range) -- the MFMA work of the busiest CU
-// -- with at most 256 workgroups per round (token groups x tiles x S); ties go to fewer
-// K ranges.  F = 0: no F divides N / 16.
+// Plan of the wide kernel: F (row tiles per workgroup, 4..9; the last tile's fragments past
+// N / 16 are padding) and the K split S that minimise the estimated time, in units of one
+// 1 KB load-to-LDS copy of a busy CU (0.022-0.025 us, whatever the operand; the light-load
+// rate is 0.02).  Fitted to every (F, S) at nine layer shapes and M = 24..256:
+//   * K blocks: (2 F + 8 TJ + 1) copies each, times the blocks of a range and the rounds of
+//     256 workgroups;
+//   * never less than the weight itself at 5.5 TB/s (7168 <-> 18432: 937 units);
+//   * a split: publishing and the counter (1.5 us; 3 us with 128-token tiles), and per range one dependent
+//     round trip of its slot (4 F TJ KB) in the last workgroup's sum.
+// Narrow layers take small tiles and few ranges (7168 -> 1536 at M = 64: F = 4, S = 6..8
+// 11.0 us; F = 6, S = 14 15.4; F = 4, S = 1 22.2), short ones none (512 -> 4096: S = 1 5.2,
+// S = 4 8.2 us).
 struct WidePlan {
   int F, TJ, TG, S, per, tiles;
   int grid() const { return static_cast<int>(cdiv(static_cast<int64_t>(tiles) * S, 8)) * 8 * TG; }
 };
 
-__host__ inline WidePlan plan_wide(int64_t M, int64_t N, int64_t K) {
-  const int NT = static_cast<int>(N / 16), KB = static_cast<int>(K / kBlock);
-  const int TJ = cdiv(M, 16) <= 4 ? 1 : 2;
-  const int TG = static_cast<int>(cdiv(cdiv(M, 16), 4 * TJ));
-  WidePlan best{0, TJ, TG, 1, KB, 0};
+__host__ inline WidePlan make_wide_plan(int M, int N, int K) {
+  const int NT = N / 16, KB = K / kBlock;
+  const int TJ = M <= 64 ? 1 : 2;
+  const int TG = (M + 64 * TJ - 1) / (64 * TJ);
+  auto up = [](int x, int y) { return (x + y - 1) / y; };
+  WidePlan best{4, TJ, TG, 1, KB, up(NT, 4)};
   int64_t best_cost = INT64_MAX;
-  for (int F = 9; F >= 4; --F) {
-    if (NT % F) continue;
-    const int tiles = NT / F;
-    int S = std::max(1, std::min(KB, kWideGrid / (tiles * TG)));
-    const int per = static_cast<int>(cdiv(KB, S));
-    S = static_cast<int>(cdiv(KB, per));
-    const int64_t cost = cdiv(static_cast<int64_t>(tiles) * TG * S, kWideGrid) * F * per * 16 + (S - 1);
-    if (cost < best_cost) { best_cost = cost; best = WidePlan{F, TJ, TG, S, per, tiles}; }
+  const int64_t floor = static_cast<int64_t>(N) * K / 141312;  // one unit's worth of HBM time at 5.5 TB/s
+  for (int F = 4; F <= 9; ++F) {
+    const int tiles = up(NT, F);
+    const int max_s = std::max(1, std::min({KB, kWideMaxSplit, kWideGrid / (tiles * TG)}));
+    for (int want = 1; want <= max_s; ++want) {
+      const int per = up(KB, want), S = up(KB, per);
+      if (S != want) continue;  // the same ranges as a smaller split
+      const int64_t split = S > 1 ? 60 * TJ + S * (10 + 4 * F * TJ) : 0;
+      if (split >= best_cost) break;
+      const int64_t work = static_cast<int64_t>(up(tiles * TG * S, kWideGrid)) * per * (2 * F + 8 * TJ + 1);
+      const int64_t cost = std::max(work, floor) + split;
+      if (cost < best_cost) { best_cost = cost; best = WidePlan{F, TJ, TG, S, per, tiles}; }
+    }
   }
   return best;
+}
+
+// A call asks for its plan several times (workspace size, offsets, launch): each thread keeps its last one.
+__host__ inline WidePlan plan_wide(int64_t M, int64_t N, int64_t K) {
+  struct Last {
+    int64_t M = 0, N = 0, K = 0;
+    WidePlan w{};
+  };
+  static thread_local Last last;
+  if (last.M != M || last.N != N || last.K != K)
+    last = Last{M, N, K, make_wide_plan(static_cast<int>(M), static_cast<int>(N), static_cast<int>(K))};
+  return last.w;
 }
 
 __host__ inline size_t wide_partial_bytes(int64_t M, int64_t N, int64_t K) {
@@ -937,77 +701,40 @@ __host__ inline size_t wide_partial_bytes(int64_t M, int64_t N, int64_t K) {
 
 
 struct GemmPlan {
-  bool mm;     // packed weight, N % 128 = 0, M > 32 (or > 16, K split <= 4): fp8_gemm_wide_kernel
-  bool tiled;  // M > 64, canonical weight: fp8_gemm_tiled_kernel
-  int ksplit;
-  int kb_per_split;
-  int row_groups;  // grid.x: 16-row tiles (GEMV) or 128-row groups (tiled)
-  int waves;
-  int depth;  // GEMV operand buffers per wave
-  int rt;     // GEMV row tiles per workgroup
-  bool xf;    // GEMV reads the activation image (act_image_kernel) from the workspace
+  bool mm;    // the wide kernel, else the GEMV:
+  int waves;  // per workgroup
+  int depth;  // operand buffers per wave
+  int rt;     // 16-row tiles per workgroup
+  bool xf;    // it reads the activation image (act_image_kernel) from the workspace
 };
 
-// K split.  GEMV (M <= 16): never split.  Measured on MI355X at every MLA, MLP and
-// MoE-sized layer, the split's extra round trips (partial store, counter, reload: ~2 us)
-// cost more than the extra CUs buy -- even a 36-tile layer, whose workgroups each stream
-// 114 KB, is faster unsplit (5.6 vs 7.7 us).  M = 17..64: a layer of fewer than 192 row
-// tiles splits K into cdiv(256, tiles) <= 4 slices of whole K groups (there the activation
-// reads make a workgroup's work long enough for the split to pay); wider layers do not.
-// Tiled (M > 64; measured faster than the per-row-tile kernel from M = 128 on, slower at
-// M = 32 and 64): the smallest split giving >= 512 workgroups (2 per CU) with slices of
-// at least 8 K blocks.
-static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, bool packed) {
+// The GEMV never splits K.  Measured on MI355X at every MLA, MLP and MoE-sized layer, the
+// split's extra round trips (partial store, counter, reload: ~2 us) cost more than the
+// extra CUs buy -- even a 36-tile layer, whose workgroups each stream 114 KB, is faster
+// unsplit (5.6 vs 7.7 us); from M = 17 on a layer narrow enough to want a split takes the
+// wide kernel.
+static GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K) {
   GemmPlan p;
   const int KB = static_cast<int>(K / kBlock);
-  p.mm = packed && N % 128 == 0 && K % (kBlock * kGroup) == 0 &&
-         (M > kWideMinM || (M > kWideMinM2 && plan_wide(M, N, K).S <= kWideMaxSplit2));
-  p.tiled = M > 64 && !p.mm;
+  const int NT = static_cast<int>(N / 16);
+  p.mm = M > kWideMinM || (M > kWideMinM2 && !(NT >= kGemvTiles0 && NT <= kGemvTiles1 && KB >= kGemvKb0 && KB <= kGemvKb1));
   p.depth = 2;
   p.rt = 1;
   p.xf = false;
-  if (p.mm) {  // the wide kernel (N % 128 = 0: F = 8 always divides N / 16)
-    p.row_groups = 0;
-    p.ksplit = 1;
-    p.kb_per_split = KB;
-    p.waves = kWideWaves;
-    p.xf = false;  // reads x [M, K] itself
-    return p;
-  }
-  if (p.tiled) {
-    p.row_groups = static_cast<int>(cdiv(N / 16, kTiledWaves));
-    int s = static_cast<int>(cdiv(512, p.row_groups));
-    s = std::max(1, std::min(s, KB / 8));
-    p.kb_per_split = static_cast<int>(cdiv(KB, s));
-    p.ksplit = static_cast<int>(cdiv(KB, p.kb_per_split));
-    p.waves = kTiledWaves;
-    return p;
-  }
-  const int groups = static_cast<int>(cdiv(KB, kGroup));
-  p.row_groups = static_cast<int>(N / 16);
-  int s = 1;
-  if (M > 16 && p.row_groups < 192) s = std::max(1, std::min({4, groups, static_cast<int>(cdiv(256, p.row_groups))}));
-  p.kb_per_split = static_cast<int>(cdiv(groups, s)) * kGroup;
-  p.ksplit = static_cast<int>(cdiv(KB, p.kb_per_split));
-  // unsplit layers: 8 waves (4 for K < 1024, where 8 would leave waves idle); split: 4
-  p.waves = (p.ksplit == 1 && KB >= 8) ? 8 : kGroup;
+  p.waves = KB >= 8 ? 8 : kGroup;  // 4 for K < 1024, where 8 would leave waves idle
+  if (p.mm) return p;
   // long, wide GEMVs keep 4 K blocks in flight per wave (measured ~1% faster on the
   // 7168 x 18432 and 18432 x 7168 layers; no gain on narrow ones)
-  if (M <= 16 && p.waves == 8 && KB >= 48 && p.row_groups >= 448) p.depth = 4;
-  // From M = 5 on, each activation fragment serves 2 or 4 row tiles (measured: up
-  // 7168 -> 18432 at M = 16 / 32 / 64: 33.2 -> 28.7 / 53.7 -> 40.8 / 103.7 -> 68.3 us; down
-  // 18432 -> 7168 at M = 16 / 64: 35.2 -> 26.8 / 103.1 -> 59.8 us; at M = 4 it is 1 us
-  // slower), keeping >= 192 workgroups; 4 row tiles only from M = 17 on (slower at 16).
-  if (M > 4 && p.ksplit == 1 && p.waves == 8) {
-    const int want = M > 16 ? 4 : 2;
-    for (int rt = want; rt > 1; rt /= 2) {
-      if (p.row_groups % rt == 0 && p.row_groups / rt >= 192) { p.rt = rt; break; }
-    }
-    if (p.rt > 1) p.depth = 2;
+  if (M <= 16 && p.waves == 8 && KB >= 48 && NT >= 448) p.depth = 4;
+  // From M = 5 on, each activation fragment serves 2 row tiles (measured: up 7168 -> 18432 at
+  // M = 16 33.2 -> 28.7 us, down 18432 -> 7168 35.2 -> 26.8; at M = 4 it is 1 us slower),
+  // keeping >= 192 workgroups.
+  if (M > 4 && p.waves == 8 && NT % 2 == 0 && NT / 2 >= 192) {
+    p.rt = 2;
+    p.depth = 2;
   }
   // The activation image costs a launch: measured worth it from M = 16 on (M = 16 up /
-  // down: 28.7 -> 27.2 / 26.7 -> 25.9 us; M = 64: 68.4 -> 51.9 / 59.9 -> 43.0 us), not at
-  // M = 8 (25.3 -> 27.7 us).
+  // down: 28.7 -> 27.2 / 26.7 -> 25.9 us), not at M = 8 (25.3 -> 27.7 us).
   p.xf = M > 16 || (M == 16 && p.rt == 2);
   return p;
 }
@@ -1021,19 +748,14 @@ constexpr size_t kCounterBytes = kWsCounterBytes;
 // Workspace: counters, then the split-K partials, then the activation image (256-aligned).
 
 static size_t image_offset(const GemmPlan& p, int64_t M, int64_t N, int64_t K) {
-  const size_t partial = p.mm ? wide_partial_bytes(M, N, K)
-                              : (p.ksplit > 1 ? static_cast<size_t>(p.ksplit) * M * N * sizeof(float) : 0);
+  const size_t partial = p.mm ? wide_partial_bytes(M, N, K) : 0;
   return kCounterBytes + (partial + 255) / 256 * 256;
 }
 
 template <bool PACKED>
 static int launch_gemm(const uint8_t* A, const float* As, const uint8_t* B, const float* Bs,
                        const OutRoute& out, int M, int N, int K, void* workspace, hipStream_t st) {
-  const GemmPlan p = plan_gemm(M, N, K, PACKED);
-  uint32_t* counters = p.ksplit > 1 ? static_cast<uint32_t*>(workspace) : nullptr;
-  float* partial = p.ksplit > 1 ? reinterpret_cast<float*>(static_cast<char*>(workspace) + kCounterBytes) : nullptr;
-  const dim3 grid(p.row_groups / p.rt, p.ksplit);
-  const int per = p.kb_per_split;
+  const GemmPlan p = plan_gemm(M, N, K);
   // From M = 16 on the activations are first rearranged into the workspace (act_image_kernel).
   const uint8_t* xa = A;
   const float* xsa = As;
@@ -1053,9 +775,9 @@ static int launch_gemm(const uint8_t* A, const float* As, const uint8_t* B, cons
     auto go = [&](auto f_tag, auto tj_tag) -> int {
       constexpr int F_ = decltype(f_tag)::value, TJ_ = decltype(tj_tag)::value;
       constexpr int lds = WideShape<F_, TJ_>::LDS;
-      const void* fn = reinterpret_cast<const void*>(fp8_gemm_wide_kernel<F_, TJ_>);
+      const void* fn = reinterpret_cast<const void*>(fp8_gemm_wide_kernel<F_, TJ_, PACKED>);
       if (const int rc = allow_dynamic_lds(fn, lds, "fp8_gemm")) return rc;
-      hipLaunchKernelGGL((fp8_gemm_wide_kernel<F_, TJ_>), dim3(w.grid()), dim3(kWideWaves * 64), lds, st, A, As, B,
+      hipLaunchKernelGGL((fp8_gemm_wide_kernel<F_, TJ_, PACKED>), dim3(w.grid()), dim3(kWideWaves * 64), lds, st, A, As, B,
                          Bs, out, part, cnt, M, N, K, w.TG, w.S, w.per);
       return check_launch("fp8_gemm");
     };
@@ -1072,25 +794,10 @@ static int launch_gemm(const uint8_t* A, const float* As, const uint8_t* B, cons
     if (w.TJ == 1) return go_f(std::integral_constant<int, 1>{});
     return go_f(std::integral_constant<int, 2>{});
   }
-  if (p.tiled) {
-    auto launch = [&](auto tt_tag) -> int {
-      constexpr int TT = decltype(tt_tag)::value;
-      const void* fn = reinterpret_cast<const void*>(fp8_gemm_tiled_kernel<TT, PACKED>);
-      if (tiled_lds_bytes<TT>() > 60 * 1024) {
-        const int rc = allow_dynamic_lds(fn, tiled_lds_bytes<TT>(), "fp8_gemm");
-        if (rc) return rc;
-      }
-      hipLaunchKernelGGL((fp8_gemm_tiled_kernel<TT, PACKED>), grid, dim3(kTiledWaves * 64), tiled_lds_bytes<TT>(), st,
-                         A, As, B, Bs, out, partial, counters, M, N, K, per);
-      return check_launch("fp8_gemm");
-    };
-    if (M <= 128) return launch(std::integral_constant<int, 8>{});
-    return launch(std::integral_constant<int, 16>{});
-  }
   auto gemv = [&](auto mt, auto w, auto d, auto rt, auto xf) {
     hipLaunchKernelGGL((fp8_gemm_kernel<decltype(mt)::value, decltype(w)::value, PACKED, decltype(d)::value,
                                         decltype(rt)::value, decltype(xf)::value>),
-                       grid, dim3(decltype(w)::value * 64), 0, st, xa, xsa, B, Bs, out, partial, counters, M, N, K, per);
+                       dim3(N / 16 / decltype(rt)::value), dim3(decltype(w)::value * 64), 0, st, xa, xsa, B, Bs, out, M, N, K);
   };
   using I1 = std::integral_constant<int, 1>;
   using I2 = std::integral_constant<int, 2>;
@@ -1098,29 +805,12 @@ static int launch_gemm(const uint8_t* A, const float* As, const uint8_t* B, cons
   using I8 = std::integral_constant<int, 8>;
   using F = std::false_type;
   using T = std::true_type;
-  // token tiles 2 or 4 (M > 16), with or without the activation image
-  auto gemv_mt = [&](auto w, auto rt) {
-    if (M <= 32) {
-      if (p.xf) gemv(I2{}, w, I2{}, rt, T{}); else gemv(I2{}, w, I2{}, rt, F{});
-    } else {
-      if (p.xf) gemv(I4{}, w, I2{}, rt, T{}); else gemv(I4{}, w, I2{}, rt, F{});
-    }
-  };
-  if (M <= 16) {
-    if (p.rt == 2 && p.xf) gemv(I1{}, I8{}, I2{}, I2{}, T{});
-    else if (p.rt == 2) gemv(I1{}, I8{}, I2{}, I2{}, F{});
-    else if (p.depth == 4) gemv(I1{}, I8{}, I4{}, I1{}, F{});
-    else if (p.waves == 8) gemv(I1{}, I8{}, I2{}, I1{}, F{});
-    else gemv(I1{}, I4{}, I2{}, I1{}, F{});
-  } else if (p.rt == 4) {
-    gemv_mt(I8{}, I4{});
-  } else if (p.rt == 2) {
-    gemv_mt(I8{}, I2{});
-  } else if (p.waves == 8) {
-    gemv_mt(I8{}, I1{});
-  } else {
-    gemv_mt(I4{}, I1{});
-  }
+  if (M > 16) gemv(I2{}, I8{}, I2{}, I1{}, T{});  // two token tiles, on the activation image
+  else if (p.rt == 2 && p.xf) gemv(I1{}, I8{}, I2{}, I2{}, T{});
+  else if (p.rt == 2) gemv(I1{}, I8{}, I2{}, I2{}, F{});
+  else if (p.depth == 4) gemv(I1{}, I8{}, I4{}, I1{}, F{});
+  else if (p.waves == 8) gemv(I1{}, I8{}, I2{}, I1{}, F{});
+  else gemv(I1{}, I4{}, I2{}, I1{}, F{});
   return check_launch("fp8_gemm");
 }
 
@@ -1262,17 +952,16 @@ __global__ __launch_bounds__(kPqWaves * 64) void rmsnorm_projq_kernel(
 
 using namespace tl;
 
-// Workspace bytes of one weight layout's plan (0 = none).
-static size_t plan_workspace_bytes(int64_t M, int64_t N, int64_t K, bool packed) {
-  const GemmPlan p = plan_gemm(M, N, K, packed);
-  if (p.ksplit > 1 || p.xf || p.mm) return image_offset(p, M, N, K) + (p.xf ? act_image_bytes(M, K) : 0);
+// Workspace bytes of the plan, which is the same for both weight layouts (0 = none).
+static size_t plan_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+  const GemmPlan p = plan_gemm(M, N, K);
+  if (p.xf || p.mm) return image_offset(p, M, N, K) + (p.xf ? act_image_bytes(M, K) : 0);
   return 0;
 }
 
 extern "C" size_t tl_fp8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0 || N % 16 || K % kBlock || M > 256) return 0;
-  // one size serves both weight layouts
-  return std::max(plan_workspace_bytes(M, N, K, false), plan_workspace_bytes(M, N, K, true));
+  return plan_workspace_bytes(M, N, K);
 }
 
 extern "C" int tl_fp8_gemm(const void* a, const float* a_s, const void* b, const float* b_s,
@@ -1422,20 +1111,52 @@ int scratch_for_current_device(void** out) {
 
 }  // namespace
 
+// Which shapes the static entry point takes is part of its interface, so it follows a fixed
+// bound and not the plans: the scratch of a K-split GEMV (M <= 64: the activation image
+// and the partials) or of a split 128-row-tile GEMM (M > 64) where N % 128 != 0 or, at M =
+// 17..32, a balanced round of 256 workgroups of 4..9 row tiles would split K more than 4 ways.
+// The plans need at most 19 MB beside the image.
+static size_t static_bound_bytes(int64_t M, int64_t N, int64_t K) {
+  const int64_t KB = K / kBlock, NT = N / 16;
+  if (N % 128 == 0 && M > 32) return 0;
+  if (N % 128 == 0 && M > 16) {
+    int64_t best = INT64_MAX, ranges = 1;
+    for (int64_t F = 9; F >= 4; --F) {
+      if (NT % F) continue;
+      const int64_t S0 = std::max<int64_t>(1, std::min<int64_t>(KB, 256 / (NT / F))), per = cdiv(KB, S0), S = cdiv(KB, per);
+      const int64_t cost = cdiv(NT / F * S, 256) * F * per * 16 + (S - 1);
+      if (cost < best) { best = cost; ranges = S; }
+    }
+    if (ranges <= 4) return 0;
+  }
+  int64_t split;
+  size_t image = 0;
+  if (M > 64) {
+    split = cdiv(KB, cdiv(KB, std::max<int64_t>(1, std::min(cdiv(512, cdiv(NT, 8)), KB / 8))));
+  } else {
+    const int64_t groups = cdiv(KB, kGroup);
+    const int64_t s = M > 16 && NT < 192 ? std::max<int64_t>(1, std::min({int64_t{4}, groups, cdiv(256, NT)})) : 1;
+    split = cdiv(KB, cdiv(groups, s) * kGroup);
+    if (M > 16 || (M == 16 && KB >= 8 && NT % 2 == 0 && NT / 2 >= 192)) image = act_image_bytes(M, K);
+  }
+  const size_t partial = split > 1 ? static_cast<size_t>(split) * M * N * sizeof(float) : 0;
+  return kCounterBytes + (partial + 255) / 256 * 256 + image;
+}
+
 extern "C" int tl_fp8_gemm_packed_static(const void* a, const float* a_s, const void* b_packed, const float* b_s,
                                          void* c_bf16, int64_t M, int64_t N, int64_t K, void* stream) {
   const char* who = "fp8_gemm_packed_static";
   if (K % (kBlock * kGroup)) { set_error("%s: K=%lld must be a multiple of 512", who, (long long)K); return kErrArg; }
   int rc = validate(who, a, a_s, b_packed, b_s, c_bf16, M, N, K, nullptr, 0, 0);
   if (rc) return rc;
-  const size_t need = plan_workspace_bytes(M, N, K, true);
+  const size_t need = std::max(plan_workspace_bytes(M, N, K), static_bound_bytes(M, N, K));
   if (need > TL_FP8_GEMM_STATIC_SCRATCH_BYTES) {
     set_error("%s: M=%lld N=%lld K=%lld needs %zu bytes of scratch, above the static maximum of %zu", who,
               (long long)M, (long long)N, (long long)K, need, static_cast<size_t>(TL_FP8_GEMM_STATIC_SCRATCH_BYTES));
     return kErrUnsupported;
   }
   void* ws = nullptr;
-  if (need) {
+  if (plan_workspace_bytes(M, N, K)) {
     rc = scratch_for_current_device(&ws);
     if (rc) return rc;
   }
