@@ -231,13 +231,6 @@ __device__ inline v8i load_kblock_stream(const uint8_t* row_kblock, int g) {
   return r;
 }
 
-__device__ inline v8i zero_v8i() {
-  v8i r;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) r[i] = 0;
-  return r;
-}
-
 // A wave-uniform float read through the vector memory path.  Scalar loads share their
 // wait counter with LDS reads, and SMEM returns out of order, so every wait on an LDS
 // read would also wait for a scalar prefetch; a vector load is counted in issue order
@@ -254,23 +247,27 @@ __host__ __device__ constexpr int vmcnt_imm(int n) { return (n & 15) | ((n >> 4)
 typedef __attribute__((address_space(3))) uint8_t* lds_u8_ptr;
 
 // Load-to-LDS copies written as inline assembly: lane l copies SIZE bytes from its own
-// global address to LDS at (wave-uniform) lds + l * SIZE.  Through the builtin, the
-// compiler cannot tell these LDS writes from the operand reads of another ring stage and
-// puts a wait for every copy in flight before each LDS read; as assembly they are
-// invisible to it, and the kernel's own s_waitcnt + s_barrier order them.
-// m0 is saved into a scratch SGPR and restored inside the statement: it is a reserved
-// register that the compiler may keep live, so the assembly leaves it as it found it.
-__device__ inline void copy_to_lds16(const void* src, uint8_t* lds) {
-  const uint32_t m0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_u8_ptr)lds)));
+// global address to LDS at `lds` (a wave-uniform 32-bit LDS address) + l * SIZE.  Through the
+// builtin, the compiler cannot tell these LDS writes from the operand reads of another
+// ring stage and puts a wait for every copy in flight before each LDS read; as assembly they
+// are invisible to it, and the kernel's own s_waitcnt (and s_barrier, where waves share a
+// stage) order them.  m0 is saved into a scratch SGPR and restored inside the statement: it is a
+// reserved register that the compiler may keep live, so the assembly leaves it as it found it.
+// NT: a non-temporal copy, for weights that are streamed once.
+template <bool NT = false>
+__device__ inline void dma_lds16(const void* src, uint32_t lds) {
   uint32_t saved;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-               : "=&s"(saved) : "v"(src), "s"(m0) : "memory");
+  if constexpr (NT)
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %1, off nt\n\ts_mov_b32 m0, %0"
+                 : "=&s"(saved) : "v"(src), "s"(__builtin_amdgcn_readfirstlane(lds)) : "memory");
+  else
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+                 : "=&s"(saved) : "v"(src), "s"(__builtin_amdgcn_readfirstlane(lds)) : "memory");
 }
-__device__ inline void copy_to_lds4(const void* src, uint8_t* lds) {
-  const uint32_t m0 = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_u8_ptr)lds)));
+__device__ inline void dma_lds4(const void* src, uint32_t lds) {
   uint32_t saved;
   asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\tglobal_load_lds_dword %1, off\n\ts_mov_b32 m0, %0"
-               : "=&s"(saved) : "v"(src), "s"(m0) : "memory");
+               : "=&s"(saved) : "v"(src), "s"(__builtin_amdgcn_readfirstlane(lds)) : "memory");
 }
 
 // Software pipeline over n items with D operand buffers: item i's loads are issued D-1

@@ -384,21 +384,6 @@ __host__ __device__ constexpr int wide_ops(int F, int TJ, int w) {
   return (2 * F - w + kWideWaves - 1) / kWideWaves + TJ + (w == 2 ? 1 : 0);
 }
 
-// Load-to-LDS copies as in copy_to_lds16 / copy_to_lds4 (common.h), but taking the LDS
-// address as a wave-uniform 32-bit value already computed, with no generic-to-LDS pointer
-// conversion per copy (m0, a reserved register, is saved and restored as there): the wide
-// kernel issues 4-8 of these per K block.
-__device__ inline void dma_lds16(const void* src, uint32_t lds) {
-  uint32_t saved;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-               : "=&s"(saved) : "v"(src), "s"(__builtin_amdgcn_readfirstlane(lds)) : "memory");
-}
-__device__ inline void dma_lds4(const void* src, uint32_t lds) {
-  uint32_t saved;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\tglobal_load_lds_dword %1, off\n\ts_mov_b32 m0, %0"
-               : "=&s"(saved) : "v"(src), "s"(__builtin_amdgcn_readfirstlane(lds)) : "memory");
-}
-
 template <int F, int TJ, bool PACKED>
 __global__ __launch_bounds__(kWideWaves * 64) void fp8_gemm_wide_kernel(
     const uint8_t* __restrict__ X, const float* __restrict__ Xs, const uint8_t* __restrict__ B,

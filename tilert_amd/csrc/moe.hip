@@ -30,7 +30,6 @@ namespace tl {
 
 constexpr int kMoeWaves = 8;        // gate/up waves per workgroup (2 workgroups per CU)
 constexpr int kDownWaves = 8;       // down waves per workgroup
-constexpr int kDownSlots = 4;  // hit experts reduced together by the down kernel
 constexpr int kDnSlots = 8;    // hit experts per batch of the LDS down kernel
 constexpr int kDownRedBytes = sizeof(float) * kDownWaves * kDnSlots * 4 * 64;  // cross-wave partials
 constexpr int kDownTermBytes = sizeof(float) * kDnSlots * 4 * 64;              // per-slot terms
@@ -312,187 +311,321 @@ __global__ __launch_bounds__(kDownWaves * 64 * TPW, 4) void moe_down_lds_kernel(
   }
 }
 
-// ---------------------------------------------------------------------- gate/up
-// Work item = (slot, 16-channel tile); a persistent grid strides over n_hit * I/16 items.
-// <= 128 VGPRs (4 waves per SIMD): two 8-wave workgroups per CU, so a 4-expert call's
-// 512 work items run in one generation
-__global__ __launch_bounds__(kMoeWaves * 64, 4) void moe_gate_up_kernel(
+// ------------------------------------------------------ larger batches
+// x [M, D] no longer fits beside the weight stream (64 KB at M = 5, D = 7168), and reading the
+// activation operands from L2 into registers costs more than the weights: 16 rows of 32-byte
+// pieces per load, a quarter of the contiguous rate.  Here every wave streams its own K
+// blocks through a private ring of two LDS stages (kBigStage: the block of two weight tiles, 4 KB,
+// and of 4 MQ tokens, MQ KB), all by load-to-LDS copies of 1 KB: a weight fragment half
+// is consecutive memory, an activation copy is 4 rows of 256 bytes.  A stage is read into
+// registers at once and refilled before its block is multiplied, so nearly both stages
+// of all 8 waves (one workgroup per CU) stay in flight, and no wave waits for another until the
+// sums of a tile are combined.  Activation chunk c of row r lands at chunk c ^ r (16 chunks
+// of 16 bytes): the operand reads of 16 rows hit 16 different chunks.  Block scales are
+// scalar loads one block ahead.
+// D = 7168, I = 2048, M = 16, 11.4 hit experts: gate/up 66.6 us (5.0 TB/s of weights), down 35.8
+// (4.7 TB/s), where the kernels with register activations and four slots a batch took
+// 75.3 and 82.3.
+constexpr int kBigWaves = 8;
+constexpr int kBigStage(int MQ) { return 4096 + MQ * 1024; }
+constexpr int kBigRing(int MQ) { return kBigWaves * 2 * kBigStage(MQ); }
+constexpr int kBigRedGu = 2 * kBigWaves * 2 * 1024;             // gate/up partials, two items
+constexpr int kBigRedDn = 2 * (kBigWaves * 2 - 2) * 1024;       // down partials, two slot pairs
+constexpr int kBigWeights = kMaxLocalExperts * 16 * 4;          // routing weights [slot][token]
+
+// Block scales through the constant address space: the copies' memory clobbers would otherwise make
+// these uniform loads vector loads, counted with the copies.
+typedef const __attribute__((address_space(4))) float* scales_ptr;
+__device__ inline scales_ptr as_scales(const float* p) { return (scales_ptr)p; }
+
+// One K block of a wave: two weight fragments, the activation operand.
+struct BigOps {
+  v8i w0, w1;
+  v8bf x[4];
+};
+
+template <int MQ>
+struct BigRing {
+  const uint8_t* base;  // this wave's stages
+  uint32_t lds;         // their LDS address
+  int lane, r, g;
+
+  __device__ inline BigRing(const uint8_t* smem, int wave, int lane_) : lane(lane_), r(lane_ & 15), g(lane_ >> 4) {
+    base = smem + wave * 2 * kBigStage(MQ);
+    lds = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_u8_ptr)base)));
+  }
+  // this lane's source in a 16-token activation block [16, ...] of row pitch `pitch` bytes (rows past M: row M - 1)
+  __device__ inline void rows(const uint8_t* x, size_t pitch, int M, const uint8_t* (&src)[MQ]) const {
+#pragma unroll
+    for (int i = 0; i < MQ; ++i) {
+      const int row = 4 * i + (lane >> 4);
+      src[i] = x + static_cast<size_t>(min(row, M - 1)) * pitch + (((lane & 15) ^ row) << 4);
+    }
+  }
+  // copies of one block into stage b: 4 + MQ (the weights, read once, leave the L2 to the activations)
+  __device__ inline void issue(const uint8_t* f0, const uint8_t* f1, const uint8_t* (&src)[MQ], size_t xoff, int b) const {
+    const uint32_t st = lds + b * kBigStage(MQ);
+    dma_lds16<true>(f0 + lane * 16, st);
+    dma_lds16<true>(f0 + 1024 + lane * 16, st + 1024);
+    dma_lds16<true>(f1 + lane * 16, st + 2048);
+    dma_lds16<true>(f1 + 1024 + lane * 16, st + 3072);
+#pragma unroll
+    for (int i = 0; i < MQ; ++i) dma_lds16(src[i] + xoff, st + 4096 + i * 1024);
+  }
+  // stage b has landed (at most the other stage's copies are in flight, none past the last block)
+  __device__ inline void wait(bool more) const {
+    if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 + MQ) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+  __device__ inline void read(int b, BigOps& o) const {
+    const uint8_t* st = base + b * kBigStage(MQ);
+    const u32x4* w = reinterpret_cast<const u32x4*>(st);
+    const u32x4 a = w[lane], c = w[64 + lane], d = w[128 + lane], e = w[192 + lane];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      o.w0[i] = a[i]; o.w0[4 + i] = c[i];
+      o.w1[i] = d[i]; o.w1[4 + i] = e[i];
+    }
+    // chunks 2g, 2g + 1, 8 + 2g, 9 + 2g of row r (rows past the copied ones: the last, their columns are not stored)
+    const int row = min(r, 4 * MQ - 1);
+    const uint8_t* xr = st + 4096 + row * 256;
+    const int ch[4] = {2 * g, 2 * g + 1, 8 + 2 * g, 9 + 2 * g};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o.x[j] = *reinterpret_cast<const v8bf*>(xr + ((ch[j] ^ row) << 4));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the stage may be refilled
+  }
+  __device__ static inline void mma(const BigOps& o, float s0, float s1, v4f& a0, v4f& a1) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      a0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(dequant8_bf16(o.w0[2 * j], o.w0[2 * j + 1], s0), o.x[j], a0, 0, 0, 0);
+      a1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(dequant8_bf16(o.w1[2 * j], o.w1[2 * j + 1], s1), o.x[j], a1, 0, 0, 0);
+    }
+  }
+};
+
+// This wave's LDS writes are visible after the barrier (its copies in flight stay in flight).
+__device__ inline void big_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Gate/up: work item = (slot, 16-channel tile), a gate and an up tile; a persistent grid of one
+// workgroup per CU strides over the items, and each wave's stream of K blocks (wave + 8 i) runs on
+// across them.  An item's partials go to one of two LDS buffers; after the barrier one
+// wave, another for each item, adds them in wave order.
+template <int MQ>
+__global__ __launch_bounds__(kBigWaves * 64, 2) void moe_gate_up_big_kernel(
     const uint16_t* __restrict__ x, const uint8_t* __restrict__ w13, const float* __restrict__ s13,
     const int32_t* __restrict__ topk_idx, int M, int topk, int e0, int n_local, int D, int I,
     uint16_t* __restrict__ h) {
-  __shared__ v4f red[kMoeWaves - 1][2][64];
+  extern __shared__ __align__(16) uint8_t smem[];
+  v4f(*red)[kBigWaves][2][64] = reinterpret_cast<v4f(*)[kBigWaves][2][64]>(smem + kBigRing(MQ));
   const uint64_t mask = routing_mask(topk_idx, M * topk, e0, n_local);
   const int n_hit = __builtin_popcountll(mask);
-  const int KB = D >> 7;
-  const int tiles = I >> 4;
-  const int rows_e = 2 * I;  // gate rows then up rows
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 15, g = lane >> 4;
-  const bool tok = r < M;
-  const uint16_t* xrow = x + static_cast<size_t>(tok ? r : 0) * D;
+  const int KB = D >> 7, tiles = I >> 4, items = n_hit * tiles;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const BigRing<MQ> ring(smem, wave, lane);
+  const uint8_t* xs[MQ];
+  ring.rows(reinterpret_cast<const uint8_t*>(x), static_cast<size_t>(D) * 2, M, xs);
+  const int n = wave < KB ? (KB - wave + kBigWaves - 1) / kBigWaves : 0;  // this wave's K blocks of an item
+  const int mine = static_cast<int>(blockIdx.x) < items ? (items - blockIdx.x + gridDim.x - 1) / gridDim.x : 0;
+  const int total = n * mine;
 
-  for (int item = blockIdx.x; item < n_hit * tiles; item += gridDim.x) {
+  struct Cursor {  // the stream's position: its item's tiles and this wave's block of it
+    const uint8_t *gate, *up;
+    scales_ptr gs, us;
+    int item, j;
+  };
+  auto at_item = [&](int item, Cursor& c) {
     const int slot = item / tiles, rt = item - slot * tiles;
     const int e = nth_set_bit(mask, slot);
-    const uint8_t* gate = w13 + (static_cast<size_t>(e) * (rows_e >> 4) + rt) * KB * 2048;
-    const uint8_t* up = gate + static_cast<size_t>(tiles) * KB * 2048;
-    const float* gs = s13 + (static_cast<size_t>(e) * (rows_e >> 7) + ((rt * 16) >> 7)) * KB;
-    const float* us = s13 + (static_cast<size_t>(e) * (rows_e >> 7) + ((I + rt * 16) >> 7)) * KB;
-    // Every operand of the next K block (both fragments, the activation block, both
-    // scales) is requested one iteration ahead.  Vector loads retire in issue order, so a
-    // current-iteration load issued after a prefetch would make the wait cover the
-    // prefetch too; here the loop body only consumes registers loaded earlier.
+    c.gate = w13 + (static_cast<size_t>(e) * (2 * tiles) + rt) * KB * 2048;
+    c.up = c.gate + static_cast<size_t>(tiles) * KB * 2048;
+    c.gs = as_scales(s13) + (static_cast<size_t>(e) * ((2 * I) >> 7) + ((rt * 16) >> 7)) * KB;
+    c.us = as_scales(s13) + (static_cast<size_t>(e) * ((2 * I) >> 7) + ((I + rt * 16) >> 7)) * KB;
+    c.item = item;
+    c.j = 0;
+  };
+  auto next = [&](Cursor& c) {
+    if (++c.j == n) at_item(min(c.item + static_cast<int>(gridDim.x), items - 1), c);
+  };
+  Cursor cur{};
+  float gs_q[2] = {0.f, 0.f}, us_q[2] = {0.f, 0.f};  // scales of the two stages
+  auto issue = [&](int b) {
+    const int kb = wave + cur.j * kBigWaves;
+    ring.issue(cur.gate + static_cast<size_t>(kb) * 2048, cur.up + static_cast<size_t>(kb) * 2048, xs,
+               static_cast<size_t>(kb) * 256, b);
+    gs_q[b] = cur.gs[kb];
+    us_q[b] = cur.us[kb];
+    next(cur);
+  };
+  if (total > 0) {
+    at_item(blockIdx.x, cur);
+    issue(0);
+    if (total > 1) issue(1);
+  }
+  int i = 0;
+  auto block = [&](int b, v4f& ag, v4f& au) {  // b: i % 2
+    BigOps o;
+    ring.wait(i + 1 < total);
+    ring.read(b, o);
+    const float gs = gs_q[b], us = us_q[b];
+    if (i + 2 < total) issue(b);
+    BigRing<MQ>::mma(o, gs, us, ag, au);
+    ++i;
+  };
+  for (int k = 0; k < mine; ++k) {
     v4f ag = {0.f, 0.f, 0.f, 0.f}, au = {0.f, 0.f, 0.f, 0.f};
-    int kb = wave;
-    v8i wg_n = zero_v8i(), wu_n = zero_v8i();
-    ActOperand xa_n = {};
-    float gs_n = 0.f, us_n = 0.f;
-    if (kb < KB) {
-      wg_n = load_fragment(gate + static_cast<size_t>(kb) * 2048, lane);
-      wu_n = load_fragment(up + static_cast<size_t>(kb) * 2048, lane);
-      xa_n = load_act(xrow + kb * kBlock, g, tok);
-      gs_n = gs[kb];
-      us_n = us[kb];
+    for (int j = 0; j < n; ++j) {
+      if (i & 1) block(1, ag, au);
+      else block(0, ag, au);
     }
-    for (; kb < KB; kb += kMoeWaves) {
-      const v8i wg = wg_n, wu = wu_n;
-      const ActOperand xa = xa_n;
-      const float gsc = gs_n, usc = us_n;
-      const int kn = kb + kMoeWaves;
-      if (kn < KB) {
-        wg_n = load_fragment(gate + static_cast<size_t>(kn) * 2048, lane);
-        wu_n = load_fragment(up + static_cast<size_t>(kn) * 2048, lane);
-        xa_n = load_act(xrow + kn * kBlock, g, tok);
-        gs_n = gs[kn];
-        us_n = us[kn];
-      }
-      ag = mfma_block_bf16(wg, gsc, xa, ag);
-      au = mfma_block_bf16(wu, usc, xa, au);
-    }
-    if (wave > 0) {
-      red[wave - 1][0][lane] = ag;
-      red[wave - 1][1][lane] = au;
-    }
-    __syncthreads();
-    if (wave == 0) {
+    const int rb = k & 1;
+    red[rb][wave][0][lane] = ag;
+    red[rb][wave][1][lane] = au;
+    big_barrier();
+    if (wave == (k & (kBigWaves - 1))) {
+      ag = red[rb][0][0][lane];
+      au = red[rb][0][1][lane];
 #pragma unroll
-      for (int w = 0; w < kMoeWaves - 1; ++w) {
-        ag += red[w][0][lane];
-        au += red[w][1][lane];
+      for (int w = 1; w < kBigWaves; ++w) {
+        ag += red[rb][w][0][lane];
+        au += red[rb][w][1][lane];
       }
-      if (tok) {
+      const int item = blockIdx.x + k * gridDim.x;
+      const int slot = item / tiles, rt = item - slot * tiles;
+      if (ring.r < M) {
         uint16_t o[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) o[j] = f32_to_bf16(silu(ag[j]) * au[j]);
-        uint16_t* dst = h + (static_cast<size_t>(slot) * M + r) * I + rt * 16 + 4 * g;
+        uint16_t* dst = h + (static_cast<size_t>(slot) * M + ring.r) * I + rt * 16 + 4 * ring.g;
         *reinterpret_cast<uint2*>(dst) = make_uint2(o[0] | (static_cast<uint32_t>(o[1]) << 16),
                                                     o[2] | (static_cast<uint32_t>(o[3]) << 16));
       }
     }
-    __syncthreads();
   }
 }
 
-// ---------------------------------------------------------------------- down + combine
-// One workgroup per 16-row output tile.  Hit experts are taken kDownSlots at a time; the
-// (slot, K block) items of a batch are dealt round-robin to the waves, each wave keeping
-// one fp32 accumulator per slot, so every wave has a weight fragment in flight for the
-// whole batch.  The per-slot partials are then reduced across waves in wave order and
-// wave 0 applies, slot by slot in ascending order, the routing weight and the per-term
-// bf16 rounding before the fp32 sum -- a fixed order, so the result is deterministic.
-__global__ __launch_bounds__(kDownWaves * 64, 4) void moe_down_kernel(
+// Down + combine: one workgroup per two 16-row output tiles, over all hit experts two slots at a time:
+// waves 0-3 take the even slot of a pair, waves 4-7 the odd one, K blocks (wave % 4) + 4 i.  A
+// pair's partials go to one of two LDS buffers; after the barrier waves 0 and 1 (one tile
+// each) add a slot's four in wave order, apply the routing weight, round the term to bf16 and add it to
+// the output in slot order, while the streams run on.
+template <int MQ>
+__global__ __launch_bounds__(kBigWaves * 64, 2) void moe_down_big_kernel(
     const uint16_t* __restrict__ h, const uint8_t* __restrict__ w2, const float* __restrict__ s2,
     const int32_t* __restrict__ topk_idx, const float* __restrict__ topk_w, int M, int topk, int e0,
     int n_local, int D, int I, uint16_t* __restrict__ y) {
-  __shared__ float red[kDownWaves][kDownSlots][4][64];
+  extern __shared__ __align__(16) uint8_t smem[];
+  constexpr int kParts = kBigWaves * 2 - 2;  // (wave, tile) partials but waves 0's and 1's own
+  v4f(*red)[kParts][64] = reinterpret_cast<v4f(*)[kParts][64]>(smem + kBigRing(MQ));
+  float(*wgt)[16] = reinterpret_cast<float(*)[16]>(smem + kBigRing(MQ) + kBigRedDn);
   const uint64_t mask = routing_mask(topk_idx, M * topk, e0, n_local);
   const int n_hit = __builtin_popcountll(mask);
   const int KB = I >> 7;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 15, g = lane >> 4;
-  const bool tok = r < M;
-  const int rt = blockIdx.x;
-  v4f yacc = {0.f, 0.f, 0.f, 0.f};
-  // one routed (expert, weight) pair per lane, loaded now and consumed by the combine:
-  // no dependent loads after the weight stream (M * topk <= 64 here; larger is looped)
-  const int pairs = M * topk;
-  const int my_e = lane_pair_expert(topk_idx, pairs, e0);
-  const float my_w = lane_pair_weight(topk_w, pairs);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int half = wave >> 2, wk = wave & 3;
+  const int rt = blockIdx.x * 2;
+  const BigRing<MQ> ring(smem, wave, lane);
+  const uint8_t* hs[MQ];
+  ring.rows(reinterpret_cast<const uint8_t*>(h), static_cast<size_t>(I) * 2, M, hs);
+  const int n = wk < KB ? (KB - wk + 3) / 4 : 0;  // this wave's K blocks of a slot
+  const int slots = (n_hit - half + 1) / 2;       // its slots: half, half + 2, ...
+  const int total = n * slots;
+  const size_t tile_bytes = static_cast<size_t>(KB) * 2048;
+  const size_t slot_bytes = static_cast<size_t>(M) * I * 2;
 
-  for (int s0 = 0; s0 < n_hit; s0 += kDownSlots) {
-    const int ns = min(kDownSlots, n_hit - s0);
-    int ex[kDownSlots];
-#pragma unroll
-    for (int j = 0; j < kDownSlots; ++j) ex[j] = j < ns ? nth_set_bit(mask, s0 + j) : 0;
-    v4f acc[kDownSlots];
-#pragma unroll
-    for (int j = 0; j < kDownSlots; ++j) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
-    const int items = ns * KB;  // item i = (slot i / KB, K block i % KB)
-    auto frag_of = [&](int it, int j) -> const uint8_t* {
-      return w2 + ((static_cast<size_t>(ex[j]) * (D >> 4) + rt) * KB + (it - j * KB)) * 2048;
-    };
-    // next item's fragment, activation block and scale are requested one iteration
-    // ahead (see the gate/up kernel for why all of them)
-    auto scale_of = [&](int it, int j) -> float {
-      return s2[(static_cast<size_t>(ex[j]) * (D >> 7) + ((rt * 16) >> 7)) * KB + (it - j * KB)];
-    };
-    auto act_of = [&](int it, int j) -> ActOperand {
-      const uint16_t* hrow = h + (static_cast<size_t>(s0 + j) * M + (tok ? r : 0)) * I;
-      return load_act(hrow + (it - j * KB) * kBlock, g, tok);
-    };
-    // Ping-pong over two operand buffers (the loop is unrolled by two) so the next item's
-    // loads are in flight during this one's MFMAs. A plain `cur = next` rotation makes the
-    // compiler copy registers at the end of each iteration, waiting for those loads.
-    struct Ops {
-      v8i w;
-      ActOperand xa;
-      float sc;
-      int j;
-    };
-    auto fetch = [&](int it, Ops& o) {
-      o.j = it / KB;
-      o.w = load_fragment(frag_of(it, o.j), lane);
-      o.xa = act_of(it, o.j);
-      o.sc = scale_of(it, o.j);
-    };
-    auto compute = [&](const Ops& o) {
-#pragma unroll
-      for (int jj = 0; jj < kDownSlots; ++jj)
-        if (jj == o.j) acc[jj] = mfma_block_bf16(o.w, o.sc, o.xa, acc[jj]);
-    };
-    constexpr int W = kDownWaves;
-    Ops b0, b1;
-    if (wave < items) fetch(wave, b0);
-    for (int it = wave; it < items; it += 2 * W) {
-      if (it + W < items) fetch(it + W, b1);
-      compute(b0);
-      if (it + W >= items) break;
-      if (it + 2 * W < items) fetch(it + 2 * W, b0);
-      compute(b1);
+  const uint8_t* f = nullptr;  // the stream's position: its slot's first tile and scales, this wave's block
+  scales_ptr sc = nullptr;
+  int cs = half, cj = 0;
+  auto at_slot = [&](int slot) {
+    const int e = nth_set_bit(mask, slot);
+    f = w2 + (static_cast<size_t>(e) * (D >> 4) + rt) * tile_bytes;
+    sc = as_scales(s2) + (static_cast<size_t>(e) * (D >> 7) + ((rt * 16) >> 7)) * KB;  // both tiles lie in one 128-row block
+  };
+  float sc_q[2] = {0.f, 0.f};
+  auto issue = [&](int b) {
+    const int kb = wk + cj * 4;
+    const uint8_t* f0 = f + static_cast<size_t>(kb) * 2048;
+    ring.issue(f0, f0 + tile_bytes, hs, cs * slot_bytes + static_cast<size_t>(kb) * 256, b);
+    sc_q[b] = sc[kb];
+    if (++cj == n) {
+      cj = 0;
+      cs += 2;
+      if (cs < n_hit) at_slot(cs);
     }
+  };
+  if (total > 0) {
+    at_slot(half);
+    issue(0);
+    if (total > 1) issue(1);
+  }
+  // routing weights [slot][token], 0 where the token does not use the expert (visible to waves 0 and 1 after
+  // the first pair's barrier)
+  for (int t = threadIdx.x; t < n_hit * 16; t += kBigWaves * 64) {
+    const int tok = t & 15, e = e0 + nth_set_bit(mask, t >> 4);
+    float w = 0.f;
+    if (tok < M)
+      for (int k = 0; k < topk; ++k)
+        if (topk_idx[tok * topk + k] == e) w = topk_w[tok * topk + k];
+    wgt[t >> 4][tok] = w;
+  }
+  v4f yacc = {0.f, 0.f, 0.f, 0.f};
+  int i = 0;
+  auto block = [&](int b, v4f& a0, v4f& a1) {
+    BigOps o;
+    ring.wait(i + 1 < total);
+    ring.read(b, o);
+    const float s = sc_q[b];
+    if (i + 2 < total) issue(b);
+    BigRing<MQ>::mma(o, s, s, a0, a1);
+    ++i;
+  };
+  for (int p = 0; 2 * p < n_hit; ++p) {
+    v4f a0 = {0.f, 0.f, 0.f, 0.f}, a1 = {0.f, 0.f, 0.f, 0.f};
+    if (2 * p + half < n_hit)
+      for (int j = 0; j < n; ++j) {
+        if (i & 1) block(1, a0, a1);
+        else block(0, a0, a1);
+      }
+    const int rb = p & 1;
+    // partial (w, t) at 2 w + t - 1 before (1, 1), - 2 after it
+    if (wave != 0) red[rb][2 * wave - (wave > 1 ? 2 : 1)][lane] = a0;
+    if (wave != 1) red[rb][2 * wave + 1 - (wave > 1 ? 2 : 1)][lane] = a1;
+    big_barrier();
+    if (wave < 2) {
+      v4f t = wave == 0 ? a0 : red[rb][0][lane];  // waves 0 and 1 of this tile: (0, 1) is partial 0, (1, 0) partial 1
+      t += wave == 0 ? red[rb][1][lane] : a1;
+      t += red[rb][2 + wave][lane];
+      t += red[rb][4 + wave][lane];
+      const float wa = wgt[2 * p][ring.r];
 #pragma unroll
-    for (int j = 0; j < kDownSlots; ++j)
+      for (int q = 0; q < 4; ++q) yacc[q] += bf16_to_f32(f32_to_bf16(t[q] * wa));
+      if (2 * p + 1 < n_hit) {
+        t = red[rb][6 + wave][lane];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) red[wave][j][q][lane] = acc[j][q];
-    __syncthreads();
-    if (wave == 0) {
-      for (int j = 0; j < ns; ++j) {
-        v4f t = {0.f, 0.f, 0.f, 0.f};
-        for (int w = 0; w < kDownWaves; ++w)
+        for (int w = 1; w < 4; ++w) t += red[rb][6 + 2 * w + wave][lane];
+        const float wb = wgt[2 * p + 1][ring.r];
 #pragma unroll
-          for (int q = 0; q < 4; ++q) t[q] += red[w][j][q][lane];
-        const float wj = routing_weight(topk_idx, topk_w, my_e, my_w, pairs, topk, e0, r, tok, ex[j]);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) yacc[q] += bf16_to_f32(f32_to_bf16(t[q] * wj));
+        for (int q = 0; q < 4; ++q) yacc[q] += bf16_to_f32(f32_to_bf16(t[q] * wb));
       }
     }
-    __syncthreads();
   }
-  if (wave == 0 && tok) {
-    uint16_t* dst = y + static_cast<size_t>(r) * D + rt * 16 + 4 * g;
+  if (wave < 2 && ring.r < M) {
+    uint16_t* dst = y + static_cast<size_t>(ring.r) * D + (rt + wave) * 16 + 4 * ring.g;
     *reinterpret_cast<uint2*>(dst) =
         make_uint2(f32_to_bf16(yacc[0]) | (static_cast<uint32_t>(f32_to_bf16(yacc[1])) << 16),
                    f32_to_bf16(yacc[2]) | (static_cast<uint32_t>(f32_to_bf16(yacc[3])) << 16));
+  }
+}
+
+// MQ = groups of 4 token rows
+template <class F>
+static int by_token_rows(int64_t M, F&& f) {
+  switch (cdiv(M, 4)) {
+    case 1: return f(std::integral_constant<int, 1>{});
+    case 2: return f(std::integral_constant<int, 2>{});
+    case 3: return f(std::integral_constant<int, 3>{});
+    default: return f(std::integral_constant<int, 4>{});
   }
 }
 
@@ -521,16 +654,25 @@ extern "C" int tl_moe_gate_up_swiglu(const void* x_bf16, const void* w13_packed,
   const int64_t max_items = n_local * (I / 16);
   const int grid = static_cast<int>(max_items < 512 ? max_items : 512);  // 2 x 8 waves per CU
   const int64_t x_bytes = M * D * 2;
-  if (x_bytes <= kLdsActBytes && M * topk <= 64) {  // activations staged in LDS, routing in lanes
+  // x staged in LDS, routing in lanes, where both fit: 2-7 % ahead of the stream with x in it at
+  // D = 4096, M = 5..8 and D = 6144, 7168, M <= 5
+  if (x_bytes <= kLdsActBytes && M * topk <= 64) {
     rc = allow_dynamic_lds(reinterpret_cast<const void*>(moe_gate_up_lds_kernel), kLdsActBytes, "moe_gate_up_swiglu");
     if (rc) return rc;
     hipLaunchKernelGGL(moe_gate_up_lds_kernel, dim3(grid), dim3(kMoeWaves * 64), static_cast<size_t>(kLdsActBytes),
                        (hipStream_t)stream, (const uint16_t*)x_bf16, (const uint8_t*)w13_packed, s13, topk_idx,
                        (int)M, (int)topk, (int)expert_begin, (int)n_local, (int)D, (int)I, (uint16_t*)h_bf16);
   } else {
-    hipLaunchKernelGGL(moe_gate_up_kernel, dim3(grid), dim3(kMoeWaves * 64), 0, (hipStream_t)stream,
-                       (const uint16_t*)x_bf16, (const uint8_t*)w13_packed, s13, topk_idx, (int)M, (int)topk,
-                       (int)expert_begin, (int)n_local, (int)D, (int)I, (uint16_t*)h_bf16);
+    auto launch = [&](auto mq_tag) -> int {
+      constexpr int MQ = decltype(mq_tag)::value, lds = kBigRing(MQ) + kBigRedGu;
+      if (const int rc2 = allow_dynamic_lds(reinterpret_cast<const void*>(moe_gate_up_big_kernel<MQ>), lds, "moe_gate_up_swiglu")) return rc2;
+      hipLaunchKernelGGL((moe_gate_up_big_kernel<MQ>), dim3(std::min<int64_t>(max_items, 256)), dim3(kBigWaves * 64), lds,
+                         (hipStream_t)stream, (const uint16_t*)x_bf16, (const uint8_t*)w13_packed, s13, topk_idx,
+                         (int)M, (int)topk, (int)expert_begin, (int)n_local, (int)D, (int)I, (uint16_t*)h_bf16);
+      return 0;
+    };
+    rc = by_token_rows(M, launch);
+    if (rc) return rc;
   }
   return check_launch("moe_gate_up_swiglu");
 }
@@ -544,7 +686,11 @@ extern "C" int tl_moe_down_combine(const void* h_bf16, const void* w2_packed, co
   if (!h_bf16 || !w2_packed || !s2 || !topk_idx || !topk_w || !y_bf16) { set_error("moe_down_combine: null pointer"); return kErrArg; }
   if ((reinterpret_cast<uintptr_t>(h_bf16) | reinterpret_cast<uintptr_t>(w2_packed)) & 15) { set_error("moe_down_combine: h and weights must be 16-byte aligned"); return kErrArg; }
   const int64_t h_bytes = M * I * 2;  // one hit expert's h rows
-  if (h_bytes <= kDnHBytes && M * topk <= 64) {  // activations staged in LDS, sb hit experts per batch
+  // Up to 5 tokens: h staged in LDS, sb hit experts per batch, two tiles' 16 waves on it; above, the
+  // batches' staging and reductions cost more than streaming h beside the weights (D = 7168, I =
+  // 2048, M = 4 / 5 / 6 / 8: 15.1 / 14.6 / 19.9 / 28.9 against 15.1 / 14.8 / 17.7 / 23.8 us;
+  // D = 6144, I = 1408: 10.9 / 11.1 / 14.6 / 21.3 against 11.7 / 11.7 / 13.9 / 18.6).
+  if (M <= 5 && h_bytes <= kDnHBytes && M * topk <= 64) {
     // (the later batches are staged through registers: kStageChunks x 16 B per thread)
     const int64_t stage_cap = (D / 16) % 2 == 0 ? 2 * kLdsActBytes : kLdsActBytes;
     const int sb = static_cast<int>(std::min<int64_t>(kDnSlots, stage_cap / h_bytes));
@@ -563,9 +709,16 @@ extern "C" int tl_moe_down_combine(const void* h_bf16, const void* w2_packed, co
     rc = (D / 16) % 2 == 0 ? launch(std::integral_constant<int, 2>{}) : launch(std::integral_constant<int, 1>{});
     if (rc) return rc;
   } else {
-    hipLaunchKernelGGL(moe_down_kernel, dim3(D / 16), dim3(kDownWaves * 64), 0, (hipStream_t)stream,
-                       (const uint16_t*)h_bf16, (const uint8_t*)w2_packed, s2, topk_idx, topk_w, (int)M, (int)topk,
-                       (int)expert_begin, (int)n_local, (int)D, (int)I, (uint16_t*)y_bf16);
+    auto launch = [&](auto mq_tag) -> int {
+      constexpr int MQ = decltype(mq_tag)::value, lds = kBigRing(MQ) + kBigRedDn + kBigWeights;
+      if (const int rc2 = allow_dynamic_lds(reinterpret_cast<const void*>(moe_down_big_kernel<MQ>), lds, "moe_down_combine")) return rc2;
+      hipLaunchKernelGGL((moe_down_big_kernel<MQ>), dim3(D / 32), dim3(kBigWaves * 64), lds, (hipStream_t)stream,
+                         (const uint16_t*)h_bf16, (const uint8_t*)w2_packed, s2, topk_idx, topk_w, (int)M, (int)topk,
+                         (int)expert_begin, (int)n_local, (int)D, (int)I, (uint16_t*)y_bf16);
+      return 0;
+    };
+    rc = by_token_rows(M, launch);
+    if (rc) return rc;
   }
   return check_launch("moe_down_combine");
 }
