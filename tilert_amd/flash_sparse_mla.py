@@ -10,7 +10,7 @@ import math
 import torch
 
 from . import _lib
-from .kernel import _require_cuda, _stream
+from .kernel import _one_device, _require_cuda, _stream
 
 MAX_SPLITS = 32
 _ARCH_ATTN = {"deepseek_v3_2": (128, 64, 40.0), "glm_5": (192, 64, None)}
@@ -65,7 +65,7 @@ def flash_sparse_mla(query: torch.Tensor, query_pe: torch.Tensor, key_value: tor
     if output.numel() != seqlen * heads * 512:
         raise ValueError("output must hold [1, seqlen, heads, 512]")
     device = query.device
-    if any(t.device != device for t in (query_pe, key_value, key_pe, indices, cur_pos, output)):
+    if not _one_device(query, query_pe, key_value, key_pe, indices, cur_pos, output):
         raise RuntimeError("flash_sparse_mla inputs must be on the same device")
     _require_cuda("flash_sparse_mla", query)
     sm = softmax_scale(model_arch) if scale is None else float(scale)

@@ -8,7 +8,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .kernel import SCALE_MODES, _require_cuda, _stream
+from .kernel import SCALE_MODES, _one_device, _require_cuda, _stream
 from .sparse_index import KI_PAGE_BYTES
 
 LN_EPS = 1e-6  # golden_forward's F.layer_norm eps (ops/layernorm_rope_rotate.py:207-213)
@@ -35,7 +35,7 @@ def _check(input_raw, cur_pos, weight, bias, freqs_cis):
     if freqs_cis.numel() != seq * 64:
         raise ValueError("freqs_cis must be the fp32 [seq, 1, 64] (cos, sin) view of the seq tokens' freqs")
     tensors = (input_raw, cur_pos, weight, bias, freqs_cis)
-    if any(t.device != input_raw.device for t in tensors):
+    if not _one_device(*tensors):
         raise ValueError("layernorm_rope_rotate inputs must be on the same device")
     if not all(t.is_contiguous() for t in tensors):
         raise ValueError("layernorm_rope_rotate inputs must be contiguous")
@@ -57,7 +57,7 @@ def layernorm_rope_rotate(input_raw: torch.Tensor, cur_pos: torch.Tensor, k_cach
         raise ValueError(f"unsupported compute_kernel_type {compute_kernel_type!r}")
     if k_cache_raw.dtype != torch.bfloat16:
         raise ValueError("k_cache must be a bfloat16 tensor.")
-    if k_cache_raw.shape[-1] != 128 or not k_cache_raw.is_contiguous() or k_cache_raw.device != input_raw.device:
+    if k_cache_raw.shape[-1] != 128 or not k_cache_raw.is_contiguous() or not _one_device(k_cache_raw, input_raw):
         raise ValueError("k_cache must be a contiguous [1, rows, 128] tensor on the input's device")
     rows = k_cache_raw.numel() // 128
     _lib.call("tl_layernorm_rope_rotate", input_raw.data_ptr(), seq, cur_pos.data_ptr(), k_cache_raw.data_ptr(),
@@ -72,7 +72,7 @@ def layernorm_rope_rotate_ki(input_raw: torch.Tensor, cur_pos: torch.Tensor, ki_
     ``layernorm_rope_rotate`` followed by ``ki_cache_write``, in one launch."""
     seq = _check(input_raw, cur_pos, weight, bias, freqs_cis)
     if ki_pages.dtype != torch.uint8 or ki_pages.dim() != 2 or ki_pages.shape[1] != KI_PAGE_BYTES \
-            or not ki_pages.is_contiguous() or ki_pages.device != input_raw.device:
+            or not ki_pages.is_contiguous() or not _one_device(ki_pages, input_raw):
         raise ValueError(f"ki_pages must be a contiguous uint8 [n_pages, {KI_PAGE_BYTES}] tensor on the input's device")
     _lib.call("tl_layernorm_rope_rotate_ki", input_raw.data_ptr(), seq, cur_pos.data_ptr(), ki_pages.data_ptr(),
               ki_pages.shape[0], weight.data_ptr(), bias.data_ptr(), freqs_cis.data_ptr(), LN_EPS,

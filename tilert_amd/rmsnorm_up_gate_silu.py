@@ -41,7 +41,9 @@ def rmsnorm_up_gate_silu(hidden_in: torch.Tensor, gamma_in: torch.Tensor, weight
         raise ValueError(f"gamma_in must be [{w.D}]")
     if hidden_out.dtype != torch.bfloat16 or hidden_out.numel() != s * w.n_local * w.I or not hidden_out.is_contiguous():
         raise ValueError(f"hidden_out must be a contiguous bfloat16 [1, s, {w.n_local}, {w.I}] tensor")
-    gamma = gamma_in.reshape(w.D).to(torch.float32).contiguous()
+    gamma = gamma_in
+    if gamma.dtype != torch.float32 or not gamma.is_contiguous():
+        gamma = gamma.reshape(w.D).to(torch.float32).contiguous()
     _require_cuda("rmsnorm_up_gate_silu", hidden_in, gamma, hidden_out, w.w13, w.s13)
     _lib.call("tl_rmsnorm_up_gate_silu", hidden_in.data_ptr(), gamma.data_ptr(), EPS[model_arch], w.w13.data_ptr(),
               w.s13.data_ptr(), s, w.n_local, w.D, w.I, hidden_out.data_ptr(), _stream(hidden_in))

@@ -22,7 +22,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .kernel import SCALE_MODES, _Workspace, _require_cuda, _stream
+from .kernel import SCALE_MODES, _Workspace, _one_device, _require_cuda, _stream
 
 _WS = _Workspace()
 
@@ -60,8 +60,7 @@ def _check(q, q_scale, kv, k_scale, weights, logits, heads=(32, 64)):
                          f"supports a head number of {' or '.join(map(str, heads))}.")
     if dim != 128 or kv.shape[-1] != 128:
         raise ValueError("dim must be 128, as we precompute scale inner kernel")
-    device = q.device
-    if any(t.device != device for t in (q_scale, kv, k_scale, weights, logits)):
+    if not _one_device(q, q_scale, kv, k_scale, weights, logits):
         raise ValueError("sparse_index inputs must be on the same device")
     _require_cuda("sparse_index", q)
     for t in (q, q_scale, kv, k_scale, weights, logits):
@@ -148,7 +147,7 @@ def _check_bf16(q, kv, weights, logits, profile_logs, extra=()):
         raise ValueError("dim must be 128, as we precompute scale inner kernel")
     device = q.device
     others = (kv, weights, logits, *extra) + ((profile_logs,) if profile_logs is not None else ())
-    if any(t.device != device for t in others):
+    if not _one_device(q, *others):
         raise ValueError("sparse_index inputs must be on the same device: "
                          f"q={device}, kv={kv.device}, weights={weights.device}, logits={logits.device}")
     _require_cuda("sparse_index", q)
