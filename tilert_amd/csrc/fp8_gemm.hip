@@ -321,10 +321,10 @@ __device__ __attribute__((always_inline)) inline void static_for(F&& f) {
 // fragment a wave reads from LDS feeds several MFMAs and each SIMD has two waves to hide
 // the other's latencies.
 // Per K block the weight fragments, the activation rows (read from x [M, K] itself) and
-// their scales are copied global -> LDS (global_load_lds, no registers) into a 4-stage
-// ring; each wave reads block i + 1's operands into a second register set while
+// their scales are copied global -> LDS (global_load_lds, no registers) into a ring of 4 to 6
+// stages; each wave reads block i + 1's operands into a second register set while
 // block i's MFMAs run.  The 2F weight pieces are dealt to the waves round robin, wave 2
-// copies the weight scales and the token scales come in 16-block windows, so per-wave copy
+// copies the weight scales and the token scales come in 8-block windows, so per-wave copy
 // counts differ, but each wave issues the same count every block (plus the window copies
 // at a window's first block, which only make the next waits stricter) and waits for its
 // own copies with a fixed s_waitcnt before the block's s_barrier.
@@ -366,19 +366,22 @@ struct WideShape {
   static constexpr int A = TT * 2048;                   // activation fragments
   static constexpr int WS = W + A;                      // weight scales (F floats)
   static constexpr int STAGE = WS + 256;
-  // Ring depth.  Deeper rings measured no faster, also for layers of few workgroups: a block's
-  // copies take the CU's address unit about 0.02 us each, which no lead hides.
-  static constexpr int STAGES = 4;
-  static constexpr int WIN = STAGES * STAGE;            // token-scale windows: [2][128][16] fp32
-  static constexpr int LDS = WIN + 2 * 128 * 16 * 4;
+  // Ring depth: as many stages as fit, at most 6.  What bounds a full chip is the copies in
+  // flight, so the 8-block scale windows that make room for a stage pay on wide layers (4 -> 5
+  // stages: 7168 -> 18432 stored at M = 33 / 64 31.2 -> 27.6 / 32.3 -> 30.2 us, 18432 -> 7168 at
+  // M = 256 58.4 -> 56.7); a layer of few workgroups gains nothing from a longer lead.
+  static constexpr int FIT = (160 * 1024 - 2 * 128 * 8 * 4 - 64) / STAGE;
+  static constexpr int STAGES = FIT < 6 ? FIT : 6;
+  static constexpr int WIN = STAGES * STAGE;            // token-scale windows: [2][128][8] fp32
+  static constexpr int LDS = WIN + 2 * 128 * 8 * 4;
   static constexpr int SLOT = F * TT * 256;             // floats of one partial
   static_assert(16 * TT <= 128, "the token-scale windows hold 128 tokens");
 };
 
 // Copy instructions wave w issues per K block: its weight pieces (the 2F 1 KB pieces dealt
 // round robin), TJ activation pieces, and the weight scales (wave 2).  At the first block
-// of each 16-block window (and of the range) waves 0 .. TT - 1 also copy their 16 tokens'
-// scales of the window (4 more copies); those blocks' waits then cover a few copies of the
+// of each 8-block window (and of the range) waves 0 .. TT - 1 also copy their 16 tokens'
+// scales of the window (2 more copies); those blocks' waits then cover a few copies of the
 // next block too, which is conservative.
 __host__ __device__ constexpr int wide_ops(int F, int TJ, int w) {
   return (2 * F - w + kWideWaves - 1) / kWideWaves + TJ + (w == 2 ? 1 : 0);
@@ -422,12 +425,11 @@ __global__ __launch_bounds__(kWideWaves * 64) void fp8_gemm_wide_kernel(
 #pragma unroll
   for (int u = 0; u < TJ; ++u)
     xa[u] = X + static_cast<size_t>(min(t0 + 16 * (4 * u + (wave >> 1)) + arow, M - 1)) * K + achunk * 16;
-  // Token scales come in 16-block windows, double-buffered in LDS as [token][16] fp32:
-  // copy u of wave w brings tokens 16 w + 4 u .. +3 of the group, 16 lanes (64 contiguous
+  // Token scales come in 8-block windows, double-buffered in LDS as [token][8] fp32:
+  // copy u of wave w brings tokens 16 w + 8 u .. +7 of the group, 8 lanes (32 contiguous
   // bytes of x_s) per token; blocks past K repeat the row's last one.
-  const int srow[4] = {min(t0 + 16 * wave + (lane >> 4), M - 1), min(t0 + 16 * wave + 4 + (lane >> 4), M - 1),
-                       min(t0 + 16 * wave + 8 + (lane >> 4), M - 1), min(t0 + 16 * wave + 12 + (lane >> 4), M - 1)};
-  const int sblk = lane & 15;
+  const int srow[2] = {min(t0 + 16 * wave + (lane >> 3), M - 1), min(t0 + 16 * wave + 8 + (lane >> 3), M - 1)};
+  const int sblk = lane & 7;
   const int fr = lane < F - 1 ? lane : F - 1;
   // weight scales (wave 2); row fragments past the weight's last one (NT not a multiple of F)
   // repeat it, here and in the pieces below, and are not stored
@@ -460,11 +462,11 @@ __global__ __launch_bounds__(kWideWaves * 64) void fp8_gemm_wide_kernel(
 #pragma unroll
     for (int u = 0; u < TJ; ++u) dma_lds16(xa[u] + kb * 128, ls + Sh::W + (wave + 8 * u) * 1024);
     if (wave == 2) dma_lds4(ws_src + kb, ls + Sh::WS);
-    if (wave < TT && ((kb & 15) == 0 || kb == kb0)) {  // the window of kb: a buffer last used 16 blocks ago
-      const int b = (kb & ~15) + sblk < KB ? (kb & ~15) + sblk : KB - 1;
-      const uint32_t win = lds0 + Sh::WIN + ((kb >> 4) & 1) * 8192 + wave * 1024;
+    if (wave < TT && ((kb & 7) == 0 || kb == kb0)) {  // the window of kb: a buffer last used 8 blocks before its first, more than the ring's lead
+      const int b = (kb & ~7) + sblk < KB ? (kb & ~7) + sblk : KB - 1;
+      const uint32_t win = lds0 + Sh::WIN + ((kb >> 3) & 1) * 4096 + wave * 512;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) dma_lds4(Xs + static_cast<size_t>(srow[u]) * KB + b, win + u * 256);
+      for (int u = 0; u < 2; ++u) dma_lds4(Xs + static_cast<size_t>(srow[u]) * KB + b, win + u * 256);
     }
   };
   // MFMA operand of a token fragment in the swizzled layout: lane (r, g) reads chunks g
@@ -503,11 +505,11 @@ __global__ __launch_bounds__(kWideWaves * 64) void fp8_gemm_wide_kernel(
       for (int j = 0; j < TJ; ++j) o.a[j] = load_act(st + Sh::W + (TJ * tp + j) * 2048);
 #pragma unroll
       for (int f = 0; f < NR; ++f) o.w[f] = PACKED ? load_fragment(st + (f0 + f) * 2048, lane) : load_act(st + (f0 + f) * 2048);
-      const float* tsr = reinterpret_cast<const float*>(smem + Sh::WIN + ((kb >> 4) & 1) * 8192) +
-                         (16 * TJ * tp + r) * 16 + (kb & 15);
+      const float* tsr = reinterpret_cast<const float*>(smem + Sh::WIN + ((kb >> 3) & 1) * 4096) +
+                         (16 * TJ * tp + r) * 8 + (kb & 7);
       const float* wsr = reinterpret_cast<const float*>(st + Sh::WS) + f0;
 #pragma unroll
-      for (int j = 0; j < TJ; ++j) o.ts[j] = tsr[256 * j];
+      for (int j = 0; j < TJ; ++j) o.ts[j] = tsr[128 * j];
 #pragma unroll
       for (int f = 0; f < NR; ++f) o.ws[f] = wsr[f];
     };
