@@ -87,7 +87,7 @@ __device__ inline float group_scale(float amax, int scale_mode) {
 // e4m3fn, RNE) where f32_to_e4m3 takes about 12 operations each.  The residuals are exact
 // while s is far from the ends of the exponent range; other scales (and infinite ones)
 // divide.  A -0 quotient loses its sign in the residual sum, hence the copysign; a NaN
-// quotient becomes -448 in the clamp, on both paths.
+// quotient becomes -448 in the clamp (v_med3's NaN rule: the smallest), on both paths.
 __device__ inline uint2 quant8_e4m3(const float (&v)[8], float s) {
   float q[8];
   if (s >= 0x1p-60f && s <= 0x1p60f) {
@@ -103,7 +103,7 @@ __device__ inline uint2 quant8_e4m3(const float (&v)[8], float s) {
     for (int i = 0; i < 8; ++i) q[i] = v[i] / s;
   }
 #pragma unroll
-  for (int i = 0; i < 8; ++i) q[i] = fminf(fmaxf(q[i], -kE4m3Max), kE4m3Max);
+  for (int i = 0; i < 8; ++i) q[i] = __builtin_amdgcn_fmed3f(q[i], -kE4m3Max, kE4m3Max);
   int lo = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], 0, false);
   lo = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], lo, true);
   int hi = __builtin_amdgcn_cvt_pk_fp8_f32(q[4], q[5], 0, false);

@@ -42,28 +42,48 @@ __device__ inline float load_w<float>(const float* p) { return *p; }
 template <>
 __device__ inline float load_w<uint16_t>(const uint16_t* p) { return bf16_to_f32(*p); }
 
-// 8 consecutive weights as fp32 (16-byte loads)
-__device__ inline void load_w8(const float* p, float (&v)[8]) {
-  const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
-  v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-  v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-}
-__device__ inline void load_w8(const uint16_t* p, float (&v)[8]) {
-  const uint4 a = *reinterpret_cast<const uint4*>(p);
-  const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+typedef uint32_t u32x4n __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2n __attribute__((ext_vector_type(2)));
+
+// A lane's 8 weights of a 128-column block row (chunk c of 16), as fp32, by non-temporal 16-byte loads whose
+// 16 lanes cover consecutive memory: bf16 columns 8c..8c+7; fp32 columns 4c..4c+3 and
+// 64+4c..+3 (8 consecutive ones would leave half of every line to the second load, which a
+// non-temporal line does not wait for: 128 us at 18432 x 7168, against 116 this way and 118 with
+// temporal loads).
+template <typename T>
+struct WChunk;
+template <>
+struct WChunk<uint16_t> {
+  static constexpr int kStep0 = 8, kOff1 = 4;  // columns: kStep0 c and kStep0 c + kOff1
+  __device__ static inline void load(const uint16_t* row, int64_t c0, int64_t, float (&v)[8]) {
+    const u32x4n a = __builtin_nontemporal_load(reinterpret_cast<const u32x4n*>(row + c0));
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    v[2 * i] = __uint_as_float(w[i] << 16);
-    v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    for (int i = 0; i < 4; ++i) {
+      v[2 * i] = __uint_as_float(a[i] << 16);
+      v[2 * i + 1] = __uint_as_float(a[i] & 0xffff0000u);
+    }
   }
-}
+};
+template <>
+struct WChunk<float> {
+  static constexpr int kStep0 = 4, kOff1 = 64;
+  __device__ static inline void load(const float* row, int64_t c0, int64_t c1, float (&v)[8]) {
+    const v4f a = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(row + c0));
+    const v4f b = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(row + c1));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[i] = a[i];
+      v[4 + i] = b[i];
+    }
+  }
+};
 
 // K % 8 == 0 and 16-byte aligned weights: HBM-bound (the weight in once, codes out).  A
 // thread holds 8 rows x 8 columns of its block in registers between the amax and the
 // encode, so the block is read once, by 16-byte loads that are all in flight together; rows
 // and chunks past the edge repeat the last one (which leaves the amax alone) and are not stored.
-// bf16 18432 x 7168 (396 MB moved): 76-100 us (4.0-5.2 TB/s) against 321 us with the
-// element-wise kernel below, which reads the block twice, two bytes a lane.
+// bf16 18432 x 7168 (396 MB moved): 64 us (6.2 TB/s; 74 with temporal loads) against 321 us
+// with the element-wise kernel below, which reads the block twice, two bytes a lane.
 template <typename T>
 __global__ __launch_bounds__(256) void weight_quant_kernel(const T* __restrict__ w, uint8_t* __restrict__ q,
                                                            float* __restrict__ s, int64_t N, int64_t K) {
@@ -71,13 +91,15 @@ __global__ __launch_bounds__(256) void weight_quant_kernel(const T* __restrict__
   constexpr int kRows = 8;  // rows per thread: r0 + 16 i
   const int64_t nb = blockIdx.y, kb = blockIdx.x;
   const int c = threadIdx.x & 15, r0 = threadIdx.x >> 4;
-  const int64_t col = kb * kBlock + 8 * c;
-  const int64_t lcol = col < K ? col : K - 8;
+  using Ch = WChunk<T>;
+  const int64_t col0 = kb * kBlock + Ch::kStep0 * c, col1 = col0 + Ch::kOff1;  // 4 columns each
   float v[kRows][8];
 #pragma unroll
   for (int i = 0; i < kRows; ++i) {
     const int64_t n = nb * kBlock + r0 + 16 * i;
-    load_w8(w + (n < N ? n : N - 1) * K + lcol, v[i]);
+    const T* row = w + (n < N ? n : N - 1) * K;
+    const int64_t tail = K - (Ch::kOff1 == 4 ? 8 : 4);  // the last whole chunk
+    Ch::load(row, col0 < K ? col0 : tail, col1 < K ? col1 : tail, v[i]);
   }
   float amax = 0.f;
 #pragma unroll
@@ -94,7 +116,12 @@ __global__ __launch_bounds__(256) void weight_quant_kernel(const T* __restrict__
   for (int i = 0; i < kRows; ++i) {
     const int64_t n = nb * kBlock + r0 + 16 * i;
     const uint2 code = quant8_e4m3(v[i], sc);
-    if (n < N && col < K) *reinterpret_cast<uint2*>(q + n * K + col) = code;
+    if constexpr (Ch::kOff1 == 4) {
+      if (n < N && col0 < K) *reinterpret_cast<uint2*>(q + n * K + col0) = code;
+    } else {
+      if (n < N && col0 < K) *reinterpret_cast<uint32_t*>(q + n * K + col0) = code.x;
+      if (n < N && col1 < K) *reinterpret_cast<uint32_t*>(q + n * K + col1) = code.y;
+    }
   }
 }
 
@@ -145,7 +172,7 @@ __device__ inline float e4m3_to_f32(uint32_t code) {
 // (4 for fp32, 8 for bf16) into one 16-byte store, so a wave stores 1 KB of consecutive memory per
 // instruction; a wave's kDqRows rows (4 apart, inside one 128-row scale block) are loaded
 // together.  v_cvt_pk_f32_fp8 decodes two codes exactly.  18432 x 7168 to fp32 (661 MB moved):
-// 108 us (6.1 TB/s) against 366 us with the one-code-per-thread kernel below, which spends its time in a
+// 96 us (6.9 TB/s; 108-122 with temporal stores) against 366 us with the one-code-per-thread kernel below, which spends its time in a
 // 64-bit division per element and moves 1 byte per lane.
 constexpr int kDqRows = 8;
 template <bool BF16>
@@ -183,9 +210,9 @@ __global__ __launch_bounds__(256) void weight_dequant_kernel(const uint8_t* __re
       uint32_t o[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) o[j] = f32_to_bf16(f[2 * j]) | (static_cast<uint32_t>(f32_to_bf16(f[2 * j + 1])) << 16);
-      *reinterpret_cast<uint4*>(static_cast<uint16_t*>(out) + n * K + col) = make_uint4(o[0], o[1], o[2], o[3]);
+      __builtin_nontemporal_store(u32x4n{o[0], o[1], o[2], o[3]}, reinterpret_cast<u32x4n*>(static_cast<uint16_t*>(out) + n * K + col));
     } else {
-      *reinterpret_cast<float4*>(static_cast<float*>(out) + n * K + col) = make_float4(f[0], f[1], f[2], f[3]);
+      __builtin_nontemporal_store(v4f{f[0], f[1], f[2], f[3]}, reinterpret_cast<v4f*>(static_cast<float*>(out) + n * K + col));
     }
   }
 }
@@ -252,6 +279,13 @@ __device__ inline float norm_factor(const float (&part)[kNormVirt / 64], int dim
 }
 
 // Normalise (and quantise) chunk c of a row: 16 consecutive lanes hold a 128-element group.
+// NT: non-temporal stores (outputs of many rows, larger than an XCD's L2 share).
+template <bool NT, class T>
+__device__ inline void store_norm(T* p, T v) {
+  if constexpr (NT) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+template <bool NT>
 __device__ inline void norm_chunk(const uint4& raw, const float (&gv)[8], float r, bool live, int c, int row, int dim,
                                   uint16_t* __restrict__ y, uint8_t* __restrict__ y8, float* __restrict__ ys,
                                   int scale_mode) {
@@ -265,7 +299,7 @@ __device__ inline void norm_chunk(const uint4& raw, const float (&gv)[8], float 
     q[2 * j] = bf16_to_f32(b[j] & 0xffff);
     q[2 * j + 1] = bf16_to_f32(b[j] >> 16);
   }
-  if (live) reinterpret_cast<uint4*>(y + static_cast<int64_t>(row) * dim)[c] = make_uint4(b[0], b[1], b[2], b[3]);
+  if (live) store_norm<NT>(reinterpret_cast<u32x4n*>(y + static_cast<int64_t>(row) * dim) + c, u32x4n{b[0], b[1], b[2], b[3]});
   if (!y8) return;  // kernel-uniform
   float amax = 0.f;
 #pragma unroll
@@ -274,7 +308,7 @@ __device__ inline void norm_chunk(const uint4& raw, const float (&gv)[8], float 
   const float sc = group_scale(amax, scale_mode);
   const uint2 code = quant8_e4m3(q, sc);
   if (live) {
-    reinterpret_cast<uint2*>(y8 + static_cast<int64_t>(row) * dim)[c] = code;
+    store_norm<NT>(reinterpret_cast<u32x2n*>(y8 + static_cast<int64_t>(row) * dim) + c, u32x2n{code.x, code.y});
     if ((c & 15) == 0) ys[static_cast<int64_t>(row) * (dim / kBlock) + (c >> 4)] = sc;
   }
 }
@@ -311,15 +345,15 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_quant_kernel(
   __syncthreads();
   const float r = norm_factor(part, dim, eps);
   const float gv[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-  norm_chunk(mine, gv, r, live, c, row, dim, y, y8, ys, scale_mode);
+  norm_chunk<false>(mine, gv, r, live, c, row, dim, y, y8, ys, scale_mode);
 }
 
 // Many rows (norm_rows_min): HBM-bound.  One workgroup takes whole rows, kept in registers between the sum and the outputs (the slices above read
 // and sum every row once per slice), strides over the rows with gamma held in registers -- as fp32
 // it is twice a row's bytes -- and requests its next row before it works on this one.  The sum is
 // the same tree: chunk tid + 256 j is virtual thread tid + 256 (j % 4)'s chunk j / 4.
-// 4096 x 7168 (147 MB moved): 34 us (4.3 TB/s) against 64 us for the slices, of which the
-// hardware conversions and the reciprocal quotient (quant8_e4m3) are 15 us.
+// 4096 x 7168 (147 MB moved): 30 us (4.9 TB/s; 34 with temporal stores) against 64 us for the
+// slices, of which the hardware conversions and the reciprocal quotient (quant8_e4m3) are 15 us.
 template <int NC>  // chunks per thread: dim <= 2048 NC
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_quant_rows_kernel(
     const uint16_t* __restrict__ x, const float* __restrict__ gamma, float eps, int rows, int dim,
@@ -355,7 +389,7 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_quant_rows_kernel(
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
       const int c = tid + j * kNormThreads;
-      norm_chunk(v[j], gv[j], r, c < nch, c, row, dim, y, y8, ys, scale_mode);
+      norm_chunk<true>(v[j], gv[j], r, c < nch, c, row, dim, y, y8, ys, scale_mode);
     }
   };
   // two rows a step, so that no row is copied between register sets; the partials alternate too:
