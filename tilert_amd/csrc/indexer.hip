@@ -522,8 +522,11 @@ __global__ __launch_bounds__(256) void ln_rope_rotate_kernel(
     const float sc = group_scale(amax, scale_mode);
     uint8_t* page = pages + (row / kKiPageKeys) * kKiPageBytes;
     const int r = static_cast<int>(row % kKiPageKeys);
-    page[r * 128 + lane] = static_cast<uint8_t>(f32_to_e4m3(fminf(fmaxf(f0 / sc, -kE4m3Max), kE4m3Max)));
-    page[r * 128 + lane + 64] = static_cast<uint8_t>(f32_to_e4m3(fminf(fmaxf(f1 / sc, -kE4m3Max), kE4m3Max)));
+    // (encoded in hardware, as quant8_e4m3: 4096 keys 4.2 -> 3.95 us; 4 keys per wave, interleaved, 5.3)
+    const int codes = __builtin_amdgcn_cvt_pk_fp8_f32(__builtin_amdgcn_fmed3f(f0 / sc, -kE4m3Max, kE4m3Max),
+                                                      __builtin_amdgcn_fmed3f(f1 / sc, -kE4m3Max, kE4m3Max), 0, false);
+    page[r * 128 + lane] = static_cast<uint8_t>(codes);
+    page[r * 128 + lane + 64] = static_cast<uint8_t>(codes >> 8);
     if (lane == 0) *reinterpret_cast<float*>(page + kKiPageKeys * 128 + r * 4) = sc;
   }
 }
