@@ -58,6 +58,12 @@ constexpr int kMaxChunks = 256;                       // per row
 constexpr int kSamplePerThread = 4;
 constexpr int kSample = kTkThreads * kSamplePerThread;  // 4096
 constexpr int kMaxRowsPerLaunch = 1024;               // arrival-counter slots
+// Rows a single workgroup holds in registers (topk_short_kernel).  Up to 8192 valid columns always (us,
+// short / chunked kernel: 4 rows of 3000 / 6000 / 8192 columns 5.4 / 11.6, 7.1 / 11.5, 7.4 / 11.4; 512 rows of
+// 4096 11.2 / 27.3); up to 16384, where 16 keys a thread spill a few registers, from 128 rows on
+// (512 rows of 16384 31 / 94, 64 rows level, 4 rows level).
+constexpr int kShortCols = 8 * kTkThreads, kShortCols16 = 16 * kTkThreads;
+constexpr int kShortRows16 = 128;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2t __attribute__((ext_vector_type(2)));
@@ -522,6 +528,41 @@ __global__ __launch_bounds__(kTkThreads) void topk_kernel(const float* __restric
   }
 }
 
+// Short rows (at most 1024 CPT valid columns): one workgroup per row holds the whole row in registers
+// and selects from it -- no sample, no candidates through memory, no arrival.  Exact and in the same
+// order, so the result is the chunked kernel's.
+template <int CPT>
+__global__ __launch_bounds__(kTkThreads) void topk_short_kernel(const float* __restrict__ logits, int64_t ld,
+                                                                int64_t valid_base, int k, int row0,
+                                                                int32_t* __restrict__ out) {
+  __shared__ TopkShared sh;
+  int slot = 0;
+  const int row = row0 + static_cast<int>(blockIdx.x);
+  const int n = row_valid(row, valid_base, ld);  // <= 1024 CPT (host)
+  int32_t* o = out + static_cast<int64_t>(row) * k;
+  if (n <= k) {  // every valid column, then -1 padding
+    for (int c = threadIdx.x; c < k; c += kTkThreads) o[c] = c < n ? c : -1;
+    return;
+  }
+  for (int i = threadIdx.x; i < kHistRows * kHistPad; i += kTkThreads) sh.hist[i] = 0u;
+  __syncthreads();
+  const float* src = logits + static_cast<int64_t>(row) * ld;
+  const int c0 = static_cast<int>(threadIdx.x) * CPT;
+  select_topk<CPT>(static_cast<uint32_t>(n), static_cast<uint32_t>(n), k, sh, slot, o,
+                   [&](uint32_t, uint64_t (&cv)[CPT]) __attribute__((always_inline)) -> uint32_t {
+    f32x4 v[CPT / 4];  // (ld is a multiple of 4: a vector that starts inside the row ends in it)
+#pragma unroll
+    for (int i = 0; i < CPT / 4; ++i) v[i] = *reinterpret_cast<const f32x4*>(src + (c0 + 4 * i < n ? c0 + 4 * i : 0));
+    uint32_t m = 0;
+#pragma unroll
+    for (int i = 0; i < CPT; ++i) {
+      cv[i] = (static_cast<uint64_t>(order_key(v[i / 4][i % 4])) << 32) | static_cast<uint32_t>(c0 + i);
+      m |= c0 + i < n ? (1u << i) : 0u;
+    }
+    return m;
+  });
+}
+
 }  // namespace tl
 
 using namespace tl;
@@ -574,6 +615,14 @@ extern "C" int tl_topk_rows(const float* logits, int64_t rows, int64_t ld, int64
   if (p.chunks < 1 || p.chunks > kMaxChunks || p.rows_per_launch < 1) {
     set_error("topk: internal plan error (chunks=%d)", p.chunks);
     return kErrUnsupported;
+  }
+  const int64_t longest = std::min<int64_t>(ld, valid_base + rows);  // valid columns of the last row
+  if (longest <= kShortCols || (longest <= kShortCols16 && rows >= kShortRows16)) {
+    auto kern = longest <= 4 * kTkThreads ? topk_short_kernel<4>
+                                          : (longest <= kShortCols ? topk_short_kernel<8> : topk_short_kernel<16>);
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(rows)), dim3(kTkThreads), 0, (hipStream_t)stream, logits, ld,
+                       valid_base, (int)k, 0, out);
+    return check_launch("topk");
   }
   const TopkWs ws = carve(workspace, rows, p.chunks);
   auto kern = p.pt == 4 ? topk_kernel<4> : topk_kernel<8>;
