@@ -139,3 +139,19 @@ def test_missing_library_fails_loudly(tmp_path):
 def test_bench_refuses_multi_gpu():
     r = subprocess.run([sys.executable, str(ROOT / "bench.py"), "--gpus", "2"], capture_output=True, text=True)
     assert r.returncode == 2 and "one GPU" in r.stderr
+
+
+def test_stream_handle_refuses_tensors_off_the_gpu(monkeypatch):
+    """pack_moe_weight has no device check before it takes the stream: a host tensor must stop there, since the
+    device index of a host tensor (-1) names the current GPU's stream and the kernel would get a host address."""
+    from tilert_amd import kernel as K
+    from tilert_amd import moe
+    launched = []
+    monkeypatch.setattr(K, "_raw_stream", lambda index: 0)
+    monkeypatch.setattr(moe._lib, "call", lambda name, *args: launched.append(name))
+    for device in ("cpu", "meta"):
+        with pytest.raises(ValueError, match="GPU"):
+            K._stream(torch.empty(1, device=device))
+    with pytest.raises(ValueError, match="GPU"):
+        moe.pack_moe_weight(torch.zeros(16, 128, dtype=torch.uint8))
+    assert not launched

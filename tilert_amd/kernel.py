@@ -20,7 +20,10 @@ _raw_stream = torch._C._cuda_getCurrentRawStream
 
 
 def _stream(t: torch.Tensor) -> int:
-    return _raw_stream(t.get_device())
+    index = t.get_device()
+    if index < 0:  # not on a GPU: as an index, -1 would name the current device's stream
+        raise ValueError(f"expected a tensor on a GPU (got {t.device})")
+    return _raw_stream(index)
 
 
 def _one_device(*ts: torch.Tensor) -> bool:
