@@ -155,3 +155,18 @@ def test_stream_handle_refuses_tensors_off_the_gpu(monkeypatch):
     with pytest.raises(ValueError, match="GPU"):
         moe.pack_moe_weight(torch.zeros(16, 128, dtype=torch.uint8))
     assert not launched
+
+
+def test_package_imports_on_a_torch_without_gpu_support():
+    """A torch built without a GPU backend lacks the raw stream function: importing must work all the same (weights
+    and checkpoints are handled on the host), and only a call that needs a GPU fails."""
+    code = ("import torch\n"
+            "if hasattr(torch._C, '_cuda_getCurrentRawStream'): del torch._C._cuda_getCurrentRawStream\n"
+            "import tilert_amd.kernel as K, tilert_amd.checkpoint, tilert_amd.sparse_index, tilert_amd.moe\n"
+            "try:\n    K.act_quant(torch.zeros(2, 128, dtype=torch.bfloat16))\n"
+            "except ValueError as e:\n    print('RAISED', e)\n"
+            "torch.cuda.current_stream = lambda i: type('S', (), {'cuda_stream': 100 + i})\n"
+            "print('HANDLE', K._raw_stream(3))\n")
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=ROOT)
+    assert "RAISED act_quant: all tensors must be on a GPU" in out.stdout, out.stderr
+    assert "HANDLE 103" in out.stdout

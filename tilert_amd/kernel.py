@@ -15,8 +15,10 @@ BLOCK = 128
 SCALE_MODES = {None: 0, "ue8m0": 1, "div": 2}
 
 
-# The current stream's handle by device index: 0.06 us a call, where building the Stream object takes 2.0
-_raw_stream = torch._C._cuda_getCurrentRawStream
+# The current stream's handle by device index: 0.06 us a call, where building the Stream object takes 2.0.
+# The function is not there in a torch without GPU support.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+    lambda index: torch.cuda.current_stream(index).cuda_stream)
 
 
 def _stream(t: torch.Tensor) -> int:
