@@ -170,3 +170,22 @@ def test_package_imports_on_a_torch_without_gpu_support():
     out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=ROOT)
     assert "RAISED act_quant: all tensors must be on a GPU" in out.stdout, out.stderr
     assert "HANDLE 103" in out.stdout
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 16, 128), (100, 18432, 640), (256, 2112, 1920), (128, 65424, 18432), (200, 65536, 640)])
+def test_gemm_calls_that_take_no_workspace(M, N, K):
+    """More than 64 tokens, N not a multiple of 128 or K not of 512, and a K or N that leaves nothing to split: a caller
+    may pass no workspace."""
+    from tilert_amd import _lib
+    assert _lib.load().tl_fp8_gemm_workspace_bytes(M, N, K) == 0
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 16, 128), (65, 128, 512), (100, 18432, 1024), (65, 592, 2048), (17, 3088, 640)])
+def test_gemm_calls_that_still_need_a_workspace(M, N, K):
+    from tilert_amd import _lib
+    lib = _lib.load()
+    need = lib.tl_fp8_gemm_workspace_bytes(M, N, K)
+    assert need > 0
+    assert lib.tl_fp8_gemm(256, 256, 256, 256, 256, M, N, K, None, 0, None) == 1
+    assert b"workspace of" in lib.tl_last_error()
+    assert lib.tl_fp8_gemm(256, 256, 256, 256, 256, M, N, K, 256, need - 1, None) == 1

@@ -6,6 +6,7 @@ import torch
 
 from oracle import reference as ref
 from tests._tol import assert_gemm_close
+from tilert_amd import _lib
 from tilert_amd import kernel as K
 from tilert_amd import synth
 
@@ -44,3 +45,21 @@ def test_wide_edges_both_layouts(cuda, M, N, Kd):
         packed = K.pack_weight(d[2], d[3])
         for _ in range(3):
             assert torch.equal(K.fp8_gemm(d[0], d[1], packed), out)
+
+
+@pytest.mark.parametrize("M,N,Kd", [(65, 16, 128), (100, 2112, 1536), (200, 4112, 1920), (129, 1040, 896)])
+def test_wide_without_a_workspace(cuda, M, N, Kd):
+    """The shapes that take no workspace run without one, stored and packed."""
+    g = synth.gen(M + N + Kd)
+    xq, xs = (t.to(cuda) for t in ref.act_quant(synth.activations(M, Kd, g)))
+    wq, ws = (t.to(cuda) for t in ref.weight_quant(torch.randn(N, Kd, generator=g) * 0.02))
+    want = ref.fp8_gemm(xq.cpu(), xs.cpu(), wq.cpu(), ws.cpu())
+    lib, st = _lib.load(), torch.cuda.current_stream(cuda).cuda_stream
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=cuda)
+    weights = [(lib.tl_fp8_gemm, wq)]
+    if Kd % 512 == 0:
+        weights.append((lib.tl_fp8_gemm_packed, K.pack_weight(wq, ws).data))
+    for fn, w in weights:
+        assert fn(xq.data_ptr(), xs.data_ptr(), w.data_ptr(), ws.data_ptr(), out.data_ptr(), M, N, Kd, None, 0, st) == 0, \
+            lib.tl_last_error()
+        assert_gemm_close(out, want, f"no workspace M={M} N={N} K={Kd}")

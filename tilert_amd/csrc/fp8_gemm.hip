@@ -644,6 +644,13 @@ struct WidePlan {
   int grid() const { return static_cast<int>(cdiv(static_cast<int64_t>(tiles) * S, 8)) * 8 * TG; }
 };
 
+// Calls of more than 64 tokens that take no workspace, which is part of the interface: N not a multiple of 128 or
+// K not of 512, with a K (below 16 blocks) or an N (more than 4088 row tiles) that leaves nothing to split.  The
+// costs below never split them (8 blocks a range at most, or more workgroups than CUs); the plan also may not.
+__host__ inline bool takes_no_workspace(int64_t M, int64_t N, int64_t K) {
+  return M > 64 && (N % 128 || K % (kBlock * kGroup)) && (K / kBlock < 16 || N / 16 > 4088);
+}
+
 __host__ inline WidePlan make_wide_plan(int M, int N, int K) {
   const int NT = N / 16, KB = K / kBlock;
   const int TJ = M <= 64 ? 1 : 2;
@@ -654,7 +661,7 @@ __host__ inline WidePlan make_wide_plan(int M, int N, int K) {
   const int64_t floor = static_cast<int64_t>(N) * K / 141312;  // one unit's worth of HBM time at 5.5 TB/s
   for (int F = 4; F <= 9; ++F) {
     const int tiles = up(NT, F);
-    const int max_s = std::max(1, std::min({KB, kWideMaxSplit, kWideGrid / (tiles * TG)}));
+    const int max_s = takes_no_workspace(M, N, K) ? 1 : std::max(1, std::min({KB, kWideMaxSplit, kWideGrid / (tiles * TG)}));
     for (int want = 1; want <= max_s; ++want) {
       const int per = up(KB, want), S = up(KB, per);
       if (S != want) continue;  // the same ranges as a smaller split
@@ -941,6 +948,7 @@ using namespace tl;
 
 // Workspace bytes of the plan, which is the same for both weight layouts (0 = none).
 static size_t plan_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+  if (takes_no_workspace(M, N, K)) return 0;
   const GemmPlan p = plan_gemm(M, N, K);
   if (p.xf || p.mm) return image_offset(p, M, N, K) + (p.xf ? act_image_bytes(M, K) : 0);
   return 0;
