@@ -51,8 +51,22 @@ def test_weight_quant_wide_equals_any(cuda, dtype, N, Kd, special):
 @pytest.mark.parametrize("N,Kd", [(1, 8), (33, 256), (130, 520), (257, 4)])
 def test_weight_dequant_wide_equals_any(cuda, dtype, N, Kd):
     """Every e4m3 code (both NaNs among them) under several scales."""
-    codes = torch.from_numpy((np.arange(N * Kd) * 37 % 256).astype(np.uint8)).reshape(N, Kd)
     s = torch.rand(-(-N // 128), -(-Kd // 128), generator=torch.Generator().manual_seed(1)) * 1e-3
+    _dequant_both_ways(cuda, dtype, N, Kd, s)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,Kd", [(1023, 1024), (1024, 1024), (2017, 520), (130, 8072), (1 << 18, 4)])
+def test_weight_dequant_from_the_wide_kernels_size(cuda, dtype, N, Kd):
+    """One row below the wide kernel's 1 M elements and at it, ragged rows and columns; the scales of every third block
+    row give results that are subnormal."""
+    s = torch.rand(-(-N // 128), -(-Kd // 128), generator=torch.Generator().manual_seed(2)) * 1e-3
+    s[::3] *= 1e-35
+    _dequant_both_ways(cuda, dtype, N, Kd, s)
+
+
+def _dequant_both_ways(cuda, dtype, N, Kd, s):
+    codes = torch.from_numpy((np.arange(N * Kd) * 37 % 256).astype(np.uint8)).reshape(N, Kd)
     q = codes.view(torch.float8_e4m3fn).to(cuda)
     old = torch.get_default_dtype()
     torch.set_default_dtype(dtype)

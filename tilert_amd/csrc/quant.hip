@@ -171,13 +171,17 @@ __device__ inline float e4m3_to_f32(uint32_t code) {
   return __uint_as_float(__float_as_uint(mag) | sign);
 }
 
-// Rows of a multiple of V columns, aligned: HBM-bound on the output.  A lane turns V codes
-// (4 for fp32, 8 for bf16) into one 16-byte store, so a wave stores 1 KB of consecutive memory per
+// Rows of a multiple of V columns, aligned, in weights of kDqWide elements: HBM-bound on the output.  A lane turns V
+// codes (4 for fp32, 8 for bf16) into one 16-byte store, so a wave stores 1 KB of consecutive memory per
 // instruction; a wave's kDqRows rows (4 apart, inside one 128-row scale block) are loaded
-// together.  v_cvt_pk_f32_fp8 decodes two codes exactly.  18432 x 7168 to fp32 (661 MB moved):
-// 96 us (6.9 TB/s; 108-122 with temporal stores) against 366 us with the one-code-per-thread kernel below, which spends its time in a
-// 64-bit division per element and moves 1 byte per lane.
+// together.  v_cvt_pk_f32_fp8 decodes two codes exactly and v_cvt_pk_bf16_f32 rounds two results (RNE): rounding in
+// integer operations made the unrolled bf16 body long enough for its instruction fetch to bound small weights
+// (512 x 2048 5.4 us, 3.6 this way).  18432 x 7168 to fp32 (661 MB moved): 96 us (6.9 TB/s) against 366 us with the
+// one-code-per-thread kernel below, which spends its time in a 64-bit division per element and moves 1 byte per lane.
 constexpr int kDqRows = 8;
+// Below 1 M elements 8 rows a lane leave too few waves (us, wide / one code per thread, bf16: 128 x 128 3.6 / 2.3,
+// 512 x 512 3.5 / 2.4, 512 x 1024 3.5 / 2.9, 1024 x 1024 3.6 / 3.8, 512 x 4096 3.7 / 5.8).
+constexpr int64_t kDqWide = 1 << 20;
 template <bool BF16>
 __global__ __launch_bounds__(256) void weight_dequant_kernel(const uint8_t* __restrict__ q, const float* __restrict__ s,
                                                              void* __restrict__ out, int64_t N, int64_t K) {
@@ -212,7 +216,7 @@ __global__ __launch_bounds__(256) void weight_dequant_kernel(const uint8_t* __re
     if constexpr (BF16) {
       uint32_t o[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) o[j] = f32_to_bf16(f[2 * j]) | (static_cast<uint32_t>(f32_to_bf16(f[2 * j + 1])) << 16);
+      for (int j = 0; j < 4; ++j) o[j] = bf16x2_bits(v2f{f[2 * j], f[2 * j + 1]});
       __builtin_nontemporal_store(u32x4n{o[0], o[1], o[2], o[3]}, reinterpret_cast<u32x4n*>(static_cast<uint16_t*>(out) + n * K + col));
     } else {
       __builtin_nontemporal_store(v4f{f[0], f[1], f[2], f[3]}, reinterpret_cast<v4f*>(static_cast<float*>(out) + n * K + col));
@@ -220,7 +224,7 @@ __global__ __launch_bounds__(256) void weight_dequant_kernel(const uint8_t* __re
   }
 }
 
-// Any K and alignment.
+// Any size, K and alignment.
 __global__ __launch_bounds__(256) void weight_dequant_any_kernel(const uint8_t* __restrict__ q,
                                                                  const float* __restrict__ s,
                                                                  void* __restrict__ out, int64_t N,
@@ -495,7 +499,7 @@ extern "C" int tl_weight_dequant(const void* q_fp8, const float* s, void* out, i
   const hipStream_t st = (hipStream_t)stream;
   const int64_t V = out_bf16 ? 8 : 4;
   const int64_t groups = cdiv(N, 4 * kDqRows);
-  if (K % V == 0 && !(reinterpret_cast<uintptr_t>(q_fp8) & (V - 1)) && !(reinterpret_cast<uintptr_t>(out) & 15) &&
+  if (N * K >= kDqWide && K % V == 0 && !(reinterpret_cast<uintptr_t>(q_fp8) & (V - 1)) && !(reinterpret_cast<uintptr_t>(out) & 15) &&
       groups <= 65535) {  // (grid.y)
     const dim3 grid(cdiv(K, 64 * V), groups);
     if (out_bf16)
