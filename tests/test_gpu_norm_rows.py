@@ -35,6 +35,14 @@ def test_rows_equal_single_rows(cuda, rows, dim, scale_fmt):
             assert torch.equal(a[i:i + 1], b), f"row {i}"
 
 
+@pytest.mark.parametrize("rows,dim,scale_fmt", [
+    (255, 8320, None), (256, 8320, "div"), (300, 10240, None), (1030, 10368, "ue8m0"), (257, 12288, None),
+    (1023, 12416, None), (1024, 12416, None), (1100, 14336, "div")])
+def test_wide_rows_equal_single_rows(cuda, rows, dim, scale_fmt):
+    """Rows of 5 to 8 slices, at the edges of the instances and of the dispatch."""
+    test_rows_equal_single_rows(cuda, rows, dim, scale_fmt)
+
+
 @pytest.mark.parametrize("dim", [128, 1536, 2048])
 def test_one_slice_rows_vs_large_batch(cuda, dim):
     """dim <= 2048 takes whole rows at every batch: any batch gives a row the same bytes."""

@@ -256,15 +256,15 @@ constexpr int kNormPerThread = kNormVirt / kNormThreads;  // virtual threads per
 constexpr int kNormMaxChunks = 2;                           // chunks per virtual thread
 constexpr int kNormSlice = kNormThreads;                    // chunks per workgroup
 constexpr int kNormMaxDim = kNormMaxChunks * kNormVirt * 8;  // 16384
-constexpr int kNormRowsGrid = 1024;  // workgroups of the whole-row kernel (4 per CU; 512 and 2048 measured level)
+constexpr int kNormRowsGrid = 1024;  // workgroups of the whole-row kernel (512 and 2048 measured level)
 // Rows from which whole rows beat slices, by slices per row: a row of one slice (dim <= 2048) is a
-// whole row either way, without the sum's clamped loads (2.5 against 2.7 us at 1 row); up
-// to 8192 wide the redundant sums of the slices cost as much as the longer chain of a whole
-// row at 256 rows (dim 7168: 128 / 256 / 512 / 4096 rows 4.6 / 5.4 / 7.5 / 34.9 us against
-// 3.7 / 5.4 / 8.5 / 49.3; dim 3072: 3.4 / 3.6 / 4.5 / 17.3 against 3.1 / 3.6 / 5.0 / 21.4);
-// beyond that the registers of a whole row leave two workgroups per CU (dim 16384: 512 / 1024 /
-// 4096 rows 16.4 / 28.4 / 88 against 15.8 / 36.2 / 189).
-__host__ inline int64_t norm_rows_min(int64_t slices) { return slices <= 1 ? 1 : (slices <= 4 ? 256 : 1024); }
+// whole row either way, without the sum's clamped loads (2.8 against 2.9 us at 1 row); up to 12288 wide the redundant
+// sums of the slices cost as much as the longer chain of a whole row at 256 rows (us, whole rows / slices; dim 7168:
+// 128 / 256 / 512 / 4096 rows 4.6 / 3.8, 5.0 / 5.2, 6.3 / 8.1, 28.5 / 48.8; dim 3072: 3.5 / 3.2, 3.7 / 3.7,
+// 4.3 / 5.0, 15.1 / 18.5; dim 12288: 5.8 / 5.2, 6.5 / 7.8, 8.7 / 11.6, 44.3 / 108); beyond that the registers of a whole
+// row (8 chunks a thread: 256 VGPRs) leave one workgroup per CU (dim 16384: 320 / 512 / 1024 / 4096 rows 13.3 / 10.7,
+// 14.7 / 14.8, 26.3 / 35.5, 78.9 / 189; dim 14336: 1024 / 4096 rows 25.6 / 24.9, 74.9 / 148).
+__host__ inline int64_t norm_rows_min(int64_t slices) { return slices <= 1 ? 1 : (slices <= 6 ? 256 : 1024); }
 
 __device__ inline float sum_squares(const uint4& raw, bool in, float ss) {
   const uint32_t w4[4] = {raw.x, raw.y, raw.z, raw.w};
@@ -361,6 +361,8 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_quant_kernel(
 // the same tree: chunk tid + 256 j is virtual thread tid + 256 (j % 4)'s chunk j / 4.
 // 4096 x 7168 (147 MB moved): 30 us (4.9 TB/s; 34 with temporal stores) against 64 us for the
 // slices, of which the hardware conversions and the reciprocal quotient (quant8_e4m3) are 15 us.
+// Instances for 1, 2, 4, 5, 6 and 8 chunks a thread: registers go with the chunks (5: 158 VGPRs, three workgroups per CU;
+// 10240 wide rows in the instance for 8 chunks, with one, 1024 / 4096 rows 23.5 / 76 us, in their own 11.7 / 39.3).
 template <int NC>  // chunks per thread: dim <= 2048 NC
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_quant_rows_kernel(
     const uint16_t* __restrict__ x, const float* __restrict__ gamma, float eps, int rows, int dim,
@@ -456,6 +458,8 @@ extern "C" int tl_rmsnorm_quant(const void* x_bf16, const float* gamma, float ep
   if (slices <= 1) launch(std::integral_constant<int, 1>{});
   else if (slices <= 2) launch(std::integral_constant<int, 2>{});
   else if (slices <= 4) launch(std::integral_constant<int, 4>{});
+  else if (slices <= 5) launch(std::integral_constant<int, 5>{});
+  else if (slices <= 6) launch(std::integral_constant<int, 6>{});
   else launch(std::integral_constant<int, 8>{});
   return check_launch("rmsnorm_quant");
 }
