@@ -37,7 +37,8 @@ def test_rows_equal_single_rows(cuda, rows, dim, scale_fmt):
 
 @pytest.mark.parametrize("rows,dim,scale_fmt", [
     (255, 8320, None), (256, 8320, "div"), (300, 10240, None), (1030, 10368, "ue8m0"), (257, 12288, None),
-    (1023, 12416, None), (1024, 12416, None), (1100, 14336, "div")])
+    (1023, 12416, None), (1024, 12416, None), (1100, 14336, "div"),
+    (1700, 8320, None), (1400, 12288, None), (2048, 7168, "ue8m0"), (7000, 2048, None)])  # plain stores: outputs above 40 MB
 def test_wide_rows_equal_single_rows(cuda, rows, dim, scale_fmt):
     """Rows of 5 to 8 slices, at the edges of the instances and of the dispatch."""
     test_rows_equal_single_rows(cuda, rows, dim, scale_fmt)

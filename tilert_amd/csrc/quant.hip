@@ -285,8 +285,17 @@ __device__ inline float norm_factor(const float (&part)[kNormVirt / 64], int dim
   return 1.0f / __builtin_sqrtf(tot / static_cast<float>(dim) + eps);
 }
 
+// Outputs (y and its codes) that the whole-row kernel stores non-temporally: between 3 and 40 MB, about what the L2s
+// hold and would write back at the kernel's end.  Smaller ones the next kernel reads from L2, and of larger ones it
+// finds in the Infinity Cache what non-temporal stores leave to memory.  us, norm + a kernel that reads the codes / that
+// reads y, non-temporal against temporal: 256 x 1536 5.4 / 5.5 against 5.2 / 5.4; 2048 x 1536 9.4 / 11.0 against
+// 10.1 / 12.2; 8192 x 1536 23.9 / 28.5 against 24.9 / 29.1; 256 x 7168 8.0 / 8.7 against 8.1 / 9.1; 1024 x 7168
+// 13.6 / 16.6 against 14.8 / 17.9; 2048 x 7168 24.0 / 30.6 against 25.0 / 29.1; 4096 x 7168 45.2 / 53.8 against
+// 43.3 / 50.9 (with 16 FP8 GEMMs 7168 -> 576 on its codes 272 against 263), though its norm alone takes 28.3 against 33.1.
+constexpr int64_t kNormNtMin = 3 << 20, kNormNtMax = 40 << 20;
+
 // Normalise (and quantise) chunk c of a row: 16 consecutive lanes hold a 128-element group.
-// NT: non-temporal stores (outputs of many rows, larger than an XCD's L2 share).
+// NT: non-temporal stores (a run-time choice between the two would be merged into one plain store).
 template <bool NT, class T>
 __device__ inline void store_norm(T* p, T v) {
   if constexpr (NT) __builtin_nontemporal_store(v, p);
@@ -359,11 +368,12 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_quant_kernel(
 // and sum every row once per slice), strides over the rows with gamma held in registers -- as fp32
 // it is twice a row's bytes -- and requests its next row before it works on this one.  The sum is
 // the same tree: chunk tid + 256 j is virtual thread tid + 256 (j % 4)'s chunk j / 4.
-// 4096 x 7168 (147 MB moved): 30 us (4.9 TB/s; 34 with temporal stores) against 64 us for the
-// slices, of which the hardware conversions and the reciprocal quotient (quant8_e4m3) are 15 us.
+// 4096 x 7168 (147 MB moved): 33 us (4.4 TB/s) against 49 us for the slices, which took 64 before the hardware
+// conversions and the reciprocal quotient (quant8_e4m3).  Up to kNormRowsGrid rows a workgroup has one row and its
+// request of a next one repeats the last row for nothing.
 // Instances for 1, 2, 4, 5, 6 and 8 chunks a thread: registers go with the chunks (5: 158 VGPRs, three workgroups per CU;
 // 10240 wide rows in the instance for 8 chunks, with one, 1024 / 4096 rows 23.5 / 76 us, in their own 11.7 / 39.3).
-template <int NC>  // chunks per thread: dim <= 2048 NC
+template <int NC, bool NT>  // chunks per thread: dim <= 2048 NC
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_quant_rows_kernel(
     const uint16_t* __restrict__ x, const float* __restrict__ gamma, float eps, int rows, int dim,
     uint16_t* __restrict__ y, uint8_t* __restrict__ y8, float* __restrict__ ys, int scale_mode) {
@@ -398,7 +408,7 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_quant_rows_kernel(
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
       const int c = tid + j * kNormThreads;
-      norm_chunk<true>(v[j], gv[j], r, c < nch, c, row, dim, y, y8, ys, scale_mode);
+      norm_chunk<NT>(v[j], gv[j], r, c < nch, c, row, dim, y, y8, ys, scale_mode);
     }
   };
   // two rows a step, so that no row is copied between register sets; the partials alternate too:
@@ -449,8 +459,11 @@ extern "C" int tl_rmsnorm_quant(const void* x_bf16, const float* gamma, float ep
     else slice(std::integral_constant<int, 2>{});
     return check_launch("rmsnorm_quant");
   }
+  const int64_t out_bytes = rows * dim * (y_fp8 ? 3 : 2);
+  const bool nt = out_bytes >= kNormNtMin && out_bytes < kNormNtMax;
   auto launch = [&](auto nc) {
-    hipLaunchKernelGGL((rmsnorm_quant_rows_kernel<decltype(nc)::value>),
+    constexpr int NC = decltype(nc)::value;
+    hipLaunchKernelGGL((nt ? rmsnorm_quant_rows_kernel<NC, true> : rmsnorm_quant_rows_kernel<NC, false>),
                        dim3(static_cast<unsigned>(rows < kNormRowsGrid ? rows : kNormRowsGrid)), dim3(kNormThreads), 0,
                        (hipStream_t)stream, (const uint16_t*)x_bf16, gamma, eps, (int)rows, (int)dim, (uint16_t*)y_bf16,
                        (uint8_t*)y_fp8, y_scale, scale_mode);
