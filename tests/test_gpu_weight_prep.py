@@ -56,7 +56,8 @@ def test_weight_dequant_wide_equals_any(cuda, dtype, N, Kd):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("N,Kd", [(1023, 1024), (1024, 1024), (2017, 520), (130, 8072), (1 << 18, 4)])
+@pytest.mark.parametrize("N,Kd", [(1023, 1024), (1024, 1024), (2017, 520), (130, 8072), (1 << 18, 4),
+                                  (9363, 7168)])  # the fp32 result is just above the 256 MB of non-temporal stores
 def test_weight_dequant_from_the_wide_kernels_size(cuda, dtype, N, Kd):
     """One row below the wide kernel's 1 M elements and at it, ragged rows and columns; the scales of every third block
     row give results that are subnormal."""
@@ -66,7 +67,7 @@ def test_weight_dequant_from_the_wide_kernels_size(cuda, dtype, N, Kd):
 
 
 def _dequant_both_ways(cuda, dtype, N, Kd, s):
-    codes = torch.from_numpy((np.arange(N * Kd) * 37 % 256).astype(np.uint8)).reshape(N, Kd)
+    codes = torch.from_numpy(np.resize((np.arange(256) * 37 % 256).astype(np.uint8), N * Kd)).reshape(N, Kd)
     q = codes.view(torch.float8_e4m3fn).to(cuda)
     old = torch.get_default_dtype()
     torch.set_default_dtype(dtype)

@@ -48,6 +48,13 @@ __device__ inline float load_w<uint16_t>(const uint16_t* p) { return bf16_to_f32
 typedef uint32_t u32x4n __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2n __attribute__((ext_vector_type(2)));
 
+// NT: a non-temporal store (a run-time choice between the two would be merged into one plain store).
+template <bool NT, class T>
+__device__ inline void store_chunk(T* p, T v) {
+  if constexpr (NT) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+
 // A lane's 8 weights of a 128-column block row (chunk c of 16), as fp32, by non-temporal 16-byte loads whose
 // 16 lanes cover consecutive memory: bf16 columns 8c..8c+7; fp32 columns 4c..4c+3 and
 // 64+4c..+3 (8 consecutive ones would leave half of every line to the second load, which a
@@ -182,7 +189,12 @@ constexpr int kDqRows = 8;
 // Below 1 M elements 8 rows a lane leave too few waves (us, wide / one code per thread, bf16: 128 x 128 3.6 / 2.3,
 // 512 x 512 3.5 / 2.4, 512 x 1024 3.5 / 2.9, 1024 x 1024 3.6 / 3.8, 512 x 4096 3.7 / 5.8).
 constexpr int64_t kDqWide = 1 << 20;
-template <bool BF16>
+// Results that the Infinity Cache cannot hold for their reader are stored non-temporally (NT).  us, dequantise + a
+// product that reads the result, NT against plain stores: bf16 2112 x 7168 (29 MB) 26.7 / 24.4, 7168 x 7168 (98 MB)
+// 50.0 / 45.2, 18432 x 7168 (252 MB) 122 / 116; fp32 7168 x 7168 (196 MB) 112 / 86, 9216 x 7168 (252 MB) 141 / 142,
+// 10240 x 7168 (280 MB) 153 / 161, 18432 x 7168 (504 MB) 269 / 275.
+constexpr int64_t kDqNtBytes = 256 << 20;
+template <bool BF16, bool NT>
 __global__ __launch_bounds__(256) void weight_dequant_kernel(const uint8_t* __restrict__ q, const float* __restrict__ s,
                                                              void* __restrict__ out, int64_t N, int64_t K) {
   constexpr int V = BF16 ? 8 : 4, W = V / 4;
@@ -217,9 +229,9 @@ __global__ __launch_bounds__(256) void weight_dequant_kernel(const uint8_t* __re
       uint32_t o[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) o[j] = bf16x2_bits(v2f{f[2 * j], f[2 * j + 1]});
-      __builtin_nontemporal_store(u32x4n{o[0], o[1], o[2], o[3]}, reinterpret_cast<u32x4n*>(static_cast<uint16_t*>(out) + n * K + col));
+      store_chunk<NT>(reinterpret_cast<u32x4n*>(static_cast<uint16_t*>(out) + n * K + col), u32x4n{o[0], o[1], o[2], o[3]});
     } else {
-      __builtin_nontemporal_store(v4f{f[0], f[1], f[2], f[3]}, reinterpret_cast<v4f*>(static_cast<float*>(out) + n * K + col));
+      store_chunk<NT>(reinterpret_cast<v4f*>(static_cast<float*>(out) + n * K + col), v4f{f[0], f[1], f[2], f[3]});
     }
   }
 }
@@ -295,12 +307,6 @@ __device__ inline float norm_factor(const float (&part)[kNormVirt / 64], int dim
 constexpr int64_t kNormNtMin = 3 << 20, kNormNtMax = 40 << 20;
 
 // Normalise (and quantise) chunk c of a row: 16 consecutive lanes hold a 128-element group.
-// NT: non-temporal stores (a run-time choice between the two would be merged into one plain store).
-template <bool NT, class T>
-__device__ inline void store_norm(T* p, T v) {
-  if constexpr (NT) __builtin_nontemporal_store(v, p);
-  else *p = v;
-}
 template <bool NT>
 __device__ inline void norm_chunk(const uint4& raw, const float (&gv)[8], float r, bool live, int c, int row, int dim,
                                   uint16_t* __restrict__ y, uint8_t* __restrict__ y8, float* __restrict__ ys,
@@ -315,7 +321,7 @@ __device__ inline void norm_chunk(const uint4& raw, const float (&gv)[8], float 
     q[2 * j] = bf16_to_f32(b[j] & 0xffff);
     q[2 * j + 1] = bf16_to_f32(b[j] >> 16);
   }
-  if (live) store_norm<NT>(reinterpret_cast<u32x4n*>(y + static_cast<int64_t>(row) * dim) + c, u32x4n{b[0], b[1], b[2], b[3]});
+  if (live) store_chunk<NT>(reinterpret_cast<u32x4n*>(y + static_cast<int64_t>(row) * dim) + c, u32x4n{b[0], b[1], b[2], b[3]});
   if (!y8) return;  // kernel-uniform
   float amax = 0.f;
 #pragma unroll
@@ -324,7 +330,7 @@ __device__ inline void norm_chunk(const uint4& raw, const float (&gv)[8], float 
   const float sc = group_scale(amax, scale_mode);
   const uint2 code = quant8_e4m3(q, sc);
   if (live) {
-    store_norm<NT>(reinterpret_cast<u32x2n*>(y8 + static_cast<int64_t>(row) * dim) + c, u32x2n{code.x, code.y});
+    store_chunk<NT>(reinterpret_cast<u32x2n*>(y8 + static_cast<int64_t>(row) * dim) + c, u32x2n{code.x, code.y});
     if ((c & 15) == 0) ys[static_cast<int64_t>(row) * (dim / kBlock) + (c >> 4)] = sc;
   }
 }
@@ -519,10 +525,10 @@ extern "C" int tl_weight_dequant(const void* q_fp8, const float* s, void* out, i
   if (N * K >= kDqWide && K % V == 0 && !(reinterpret_cast<uintptr_t>(q_fp8) & (V - 1)) && !(reinterpret_cast<uintptr_t>(out) & 15) &&
       groups <= 65535) {  // (grid.y)
     const dim3 grid(cdiv(K, 64 * V), groups);
-    if (out_bf16)
-      hipLaunchKernelGGL(weight_dequant_kernel<true>, grid, dim3(256), 0, st, (const uint8_t*)q_fp8, s, out, N, K);
-    else
-      hipLaunchKernelGGL(weight_dequant_kernel<false>, grid, dim3(256), 0, st, (const uint8_t*)q_fp8, s, out, N, K);
+    const bool nt = N * K * (out_bf16 ? 2 : 4) > kDqNtBytes;
+    const auto kern = out_bf16 ? (nt ? weight_dequant_kernel<true, true> : weight_dequant_kernel<true, false>)
+                               : (nt ? weight_dequant_kernel<false, true> : weight_dequant_kernel<false, false>);
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (const uint8_t*)q_fp8, s, out, N, K);
   } else {
     hipLaunchKernelGGL(weight_dequant_any_kernel, dim3(cdiv(N * K, 256)), dim3(256), 0, st, (const uint8_t*)q_fp8, s,
                        out, N, K, out_bf16);
