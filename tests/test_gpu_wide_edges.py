@@ -25,6 +25,8 @@ pytestmark = pytest.mark.gpu
     (24, 3072, 1024),   # the GEMV's range at M = 17..32
     (32, 4096, 4096),
     (24, 4112, 1024),   # one row tile past it
+    (24, 3072, 5120),   # the longest of the GEMV's range, and a block past it
+    (24, 3072, 5248),
     (40, 18448, 512),   # more row tiles than one round of the smallest tile
 ])
 def test_wide_edges_both_layouts(cuda, M, N, Kd):

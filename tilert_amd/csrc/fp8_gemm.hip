@@ -339,14 +339,17 @@ __device__ __attribute__((always_inline)) inline void static_for(F&& f) {
 // Against the GEMV (us, wide / GEMV, packed): from M = 33 on always (7168 -> 18432 / 1536 /
 // 576 at M = 64: 29.8 / 49.8, 11.7 / 22.9, 10.3 / 15.0; 512 -> 4096 5.0 / 5.9; 1536 -> 3072
 // level); at M = 17..32 but for layers whose 16-row tiles give the GEMV one workgroup on
-// 192..256 CUs with no K split and a short stream (1536 -> 3072 at M = 24: 7.7 / 6.2;
-// 2048 -> 4096 9.6 / 6.8; 4096 -> 4096 11.0 / 9.1; next to them 2048 -> 2048 8.3 / 9.3 and
-// 4096 -> 5120 10.5 / 12.3; 512 -> 4096 4.9 / 5.3); at M <= 16 never (7168 -> 18432 at M = 16
-// 28.3 / 26.9, 7168 -> 1536 11.8 / 8.3).
+// 192..256 CUs and a stream of 8..40 K blocks (M = 24, packed: 1536 -> 3072 7.7 / 6.6, 2048 -> 4096 9.6 / 7.1,
+// 4096 -> 4096 11.0 / 9.1, 5120 -> 3072 11.6 / 9.7, 6144 -> 3072 11.2 / 10.7, 7168 -> 3072 11.7 / 11.9).  As stored the
+// GEMV's rows cost it more: 4096 -> 3072 10.0 / 10.0, 5120 -> 3072 11.2 / 11.9, 6144 -> 3072 11.1 / 12.7, which with the
+// packed weights' draws the line at 40.  A 257th tile is a second round for the GEMV (2048 -> 4112: packed
+// 8.7 / 7.8, stored 8.5 / 9.4); narrower layers of 12..20 blocks would gain from it too (2048 -> 2112: packed 8.7 / 6.9,
+// stored 8.5 / 7.7) but lose at other lengths as stored (5120 -> 2112 10.5 / 11.7).  At M <= 16 never (7168 -> 18432
+// at M = 16 28.3 / 26.9, 7168 -> 1536 11.8 / 8.3).
 constexpr int kWideMinM = 32;   // from M = 33 on always
 constexpr int kWideMinM2 = 16;  // from M = 17 on but for
 constexpr int kGemvTiles0 = 192, kGemvTiles1 = 256;  // 16-row tiles and
-constexpr int kGemvKb0 = 8, kGemvKb1 = 32;           // K blocks in these ranges
+constexpr int kGemvKb0 = 8, kGemvKb1 = 40;           // K blocks in these ranges
 constexpr int kWideMaxSplit = 32;  // K ranges
 constexpr int kWideGrid = 256;
 constexpr int kCpolSc1 = 16;            // buffer access cache policy: sc1
