@@ -1,6 +1,7 @@
-"""The MoE kernels that stream their activations beside the weights (larger batches): every group of 4
-tokens, K shorter than a workgroup's waves and not a multiple of them, odd and even hit counts, one and
-many experts, more than 64 routed pairs, repeated expert ids."""
+"""The MoE kernels beyond the small batches' LDS ones, and the edges between them: the ones that stream their
+activations beside the weights with every group of 4 tokens, the register gate/up of small layers, K shorter than a
+workgroup's waves and not a multiple of them, odd and even hit counts, one and many experts, more than 64 routed
+pairs, repeated expert ids."""
 import pytest
 import torch
 
@@ -58,3 +59,42 @@ def test_moe_batch_no_hits_and_repeated_ids(cuda):
     a, _, _ = _run(6, 4, 256, 256, 3, 32, 0, seed=4, idx=ids, w=w)
     b, _, _ = _run(6, 4, 256, 256, 3, 32, 0, seed=4, idx=torch.tensor([[30, 2, 1]] * 6, dtype=torch.int32), w=w)
     assert torch.equal(a, b)
+
+
+def _coded(E, N, K, g):
+    """Stacked e4m3fn weights [E, N, K] and scales, made as codes."""
+    q = (torch.randn(E, N, K, generator=g, device="cuda", dtype=torch.bfloat16) * 112).clamp_(-448, 448)
+    s = (torch.rand(E, N // 128, K // 128, generator=g, device="cuda") + 0.5) * 2e-4
+    return q.to(torch.float8_e4m3fn), s
+
+
+@pytest.mark.parametrize("M,E,D,I,topk,n_exp", [
+    # gate/up: the streaming kernel's four groups of 4 tokens (M = 4 by its 68 pairs, and by x above 64 KB)
+    (3, 32, 2176, 1792, 22, 96), (4, 32, 2176, 1408, 17, 96), (4, 16, 8320, 2688, 8, 128),
+    (8, 32, 2176, 768, 9, 96), (12, 16, 2176, 896, 6, 64), (16, 16, 2176, 768, 5, 64),
+    # its neighbours in the register kernel: D and the number of work items just inside its limits
+    (16, 16, 1024, 1408, 5, 64), (13, 16, 2048, 1408, 5, 64), (16, 16, 2176, 640, 5, 64),
+    # down at 6 to 8 tokens: h of 1, 2, 5 and 6 K blocks staged in LDS, of 3, 4 and 9 streamed
+    (6, 8, 256, 128, 8, 32), (7, 8, 256, 256, 8, 32), (8, 8, 384, 640, 8, 32), (6, 8, 256, 768, 8, 32),
+    (6, 8, 256, 384, 8, 32), (8, 8, 384, 512, 8, 32), (7, 8, 256, 1152, 8, 32), (9, 8, 256, 640, 7, 32),
+])
+def test_moe_dispatch_edges(cuda, M, E, D, I, topk, n_exp):
+    g = torch.Generator(device=cuda).manual_seed(M * 1000 + E + D + I)
+    gate, up, down = _coded(E, I, D, g), _coded(E, I, D, g), _coded(E, D, I, g)
+    h_ = synth.gen(M + D)
+    x, (idx, w) = synth.activations(M, D, h_), synth.routing(M, n_exp, topk, h_)
+    ex = moe.LocalExperts(*gate, *up, *down)
+    h = moe.ep_gate_up_swiglu(x.to(cuda), idx.to(cuda), ex)
+    y = moe.ep_down_combine(h, ex, idx.to(cuda), w.to(cuda))
+    hits = ref.hit_experts(idx, 0, E)
+    cpu = [[t[hits].cpu() for t in pair] for pair in (gate, up, down)]
+    slot = torch.full((n_exp,), -1, dtype=torch.int32)
+    slot[torch.tensor(hits)] = torch.arange(len(hits), dtype=torch.int32)
+    ids = slot[idx.long()]  # the hit experts renumbered 0, 1, ...
+    rh, rhits = ref.moe_gate_up(x, *cpu[0], *cpu[1], ids, 0)
+    assert rhits == list(range(len(hits)))
+    assert_gemm_close(h[:len(hits)], rh, "gate/up")
+    assert_gemm_close(y, ref.moe_down(h[:len(hits)].cpu(), rhits, *cpu[2], ids, w, 0), "down")
+    for _ in range(2):
+        assert torch.equal(moe.ep_gate_up_swiglu(x.to(cuda), idx.to(cuda), ex)[:len(hits)], h[:len(hits)])
+        assert torch.equal(moe.ep_down_combine(h, ex, idx.to(cuda), w.to(cuda)), y)

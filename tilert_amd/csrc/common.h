@@ -231,6 +231,13 @@ __device__ inline v8i load_kblock_stream(const uint8_t* row_kblock, int g) {
   return r;
 }
 
+__device__ inline v8i zero_v8i() {
+  v8i r;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) r[i] = 0;
+  return r;
+}
+
 // A wave-uniform float read through the vector memory path.  Scalar loads share their
 // wait counter with LDS reads, and SMEM returns out of order, so every wait on an LDS
 // read would also wait for a scalar prefetch; a vector load is counted in issue order

@@ -197,6 +197,88 @@ __global__ __launch_bounds__(kMoeWaves * 64, 4) void moe_gate_up_lds_kernel(
   if (!staged) __builtin_amdgcn_s_waitcnt(0);  // no item: the LDS copies land before the workgroup ends
 }
 
+// ------------------------------------------------------ gate/up, register activations
+// Small layers whose x or routing the LDS kernel above does not hold (gate_up_from_registers): work items, reduction
+// and output are the same, the activation operands come from L2.  <= 128 VGPRs (4 waves per SIMD): two workgroups
+// per CU where the kernel of the larger batches below has one; with few items, or little K, that one's longer start
+// and its rounds of 256 items cost more than the activation loads here.
+__global__ __launch_bounds__(kMoeWaves * 64, 4) void moe_gate_up_kernel(
+    const uint16_t* __restrict__ x, const uint8_t* __restrict__ w13, const float* __restrict__ s13,
+    const int32_t* __restrict__ topk_idx, int M, int topk, int e0, int n_local, int D, int I,
+    uint16_t* __restrict__ h) {
+  __shared__ v4f red[kMoeWaves - 1][2][64];
+  const uint64_t mask = routing_mask(topk_idx, M * topk, e0, n_local);
+  const int n_hit = __builtin_popcountll(mask);
+  const int KB = D >> 7;
+  const int tiles = I >> 4;
+  const int rows_e = 2 * I;  // gate rows then up rows
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const bool tok = r < M;
+  const uint16_t* xrow = x + static_cast<size_t>(tok ? r : 0) * D;
+
+  for (int item = blockIdx.x; item < n_hit * tiles; item += gridDim.x) {
+    const int slot = item / tiles, rt = item - slot * tiles;
+    const int e = nth_set_bit(mask, slot);
+    const uint8_t* gate = w13 + (static_cast<size_t>(e) * (rows_e >> 4) + rt) * KB * 2048;
+    const uint8_t* up = gate + static_cast<size_t>(tiles) * KB * 2048;
+    const float* gs = s13 + (static_cast<size_t>(e) * (rows_e >> 7) + ((rt * 16) >> 7)) * KB;
+    const float* us = s13 + (static_cast<size_t>(e) * (rows_e >> 7) + ((I + rt * 16) >> 7)) * KB;
+    // Every operand of the next K block (both fragments, the activation block, both
+    // scales) is requested one iteration ahead.  Vector loads retire in issue order, so a
+    // current-iteration load issued after a prefetch would make the wait cover the
+    // prefetch too; here the loop body only consumes registers loaded earlier.
+    v4f ag = {0.f, 0.f, 0.f, 0.f}, au = {0.f, 0.f, 0.f, 0.f};
+    int kb = wave;
+    v8i wg_n = zero_v8i(), wu_n = zero_v8i();
+    ActOperand xa_n = {};
+    float gs_n = 0.f, us_n = 0.f;
+    if (kb < KB) {
+      wg_n = load_fragment(gate + static_cast<size_t>(kb) * 2048, lane);
+      wu_n = load_fragment(up + static_cast<size_t>(kb) * 2048, lane);
+      xa_n = load_act(xrow + kb * kBlock, g, tok);
+      gs_n = gs[kb];
+      us_n = us[kb];
+    }
+    for (; kb < KB; kb += kMoeWaves) {
+      const v8i wg = wg_n, wu = wu_n;
+      const ActOperand xa = xa_n;
+      const float gsc = gs_n, usc = us_n;
+      const int kn = kb + kMoeWaves;
+      if (kn < KB) {
+        wg_n = load_fragment(gate + static_cast<size_t>(kn) * 2048, lane);
+        wu_n = load_fragment(up + static_cast<size_t>(kn) * 2048, lane);
+        xa_n = load_act(xrow + kn * kBlock, g, tok);
+        gs_n = gs[kn];
+        us_n = us[kn];
+      }
+      ag = mfma_block_bf16(wg, gsc, xa, ag);
+      au = mfma_block_bf16(wu, usc, xa, au);
+    }
+    if (wave > 0) {
+      red[wave - 1][0][lane] = ag;
+      red[wave - 1][1][lane] = au;
+    }
+    __syncthreads();
+    if (wave == 0) {
+#pragma unroll
+      for (int w = 0; w < kMoeWaves - 1; ++w) {
+        ag += red[w][0][lane];
+        au += red[w][1][lane];
+      }
+      if (tok) {
+        uint16_t o[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = f32_to_bf16(silu(ag[j]) * au[j]);
+        uint16_t* dst = h + (static_cast<size_t>(slot) * M + r) * I + rt * 16 + 4 * g;
+        *reinterpret_cast<uint2*>(dst) = make_uint2(o[0] | (static_cast<uint32_t>(o[1]) << 16),
+                                                    o[2] | (static_cast<uint32_t>(o[3]) << 16));
+      }
+    }
+    __syncthreads();
+  }
+}
+
 // ------------------------------------------------------ down, LDS activations
 // Used when one hit expert's h rows [M, I] fit in 64 KB.  A workgroup covers TPW 16-row
 // output tiles with 8 waves each, so the staged h rows serve TPW tiles.  Hit experts are
@@ -629,6 +711,18 @@ static int by_token_rows(int64_t M, F&& f) {
   }
 }
 
+// Gate/up of x or routing that the LDS kernel does not hold: the register kernel up to these sizes, else the kernel of
+// the larger batches.  n_local I M stands for the number of work items (us, register / larger batches, 8 experts of 256
+// a token; 32 local: D = 512, I = 512, M = 16 5.4 / 6.2; D = 1024, I = 2048, M = 16 14.8 / 16.2; D = 2048, I = 1024, M = 10
+// 11.5 / 12.7, M = 14 14.7 / 15.1, M = 16 15.5 / 15.0; D = 2048, I = 2048, M = 10 18.9 / 21.0, M = 14 23.9 / 23.7; D = 4096,
+// I = 512, M = 9 10.1 / 10.7, M = 14 level; D = 7168, I = 512, M = 8 12.1 / 12.4, M = 12 19.0 / 18.3; D = 7168, I = 1024, M = 6
+// 20.7 / 20.3; 16 local: D = 4096, I = 512, M = 11 8.7 / 9.2; D = 6144, I = 768, M = 9 10.5 / 11.1; D = 7168, I = 1024, M = 10
+// 0.98).
+static bool gate_up_from_registers(int64_t M, int64_t n_local, int64_t D, int64_t I) {
+  const int64_t items = n_local * I * M;
+  return D <= 1024 || (D <= 2048 && (M < 14 || items <= 1 << 19)) || items <= 5 << 15;
+}
+
 static int check_moe(const char* who, int64_t M, int64_t topk, int64_t n_local, int64_t D, int64_t I) {
   if (M < 1 || M > 16) { set_error("%s: M=%lld must be in [1, 16]", who, (long long)M); return kErrUnsupported; }
   if (topk < 1 || topk > 64) { set_error("%s: topk=%lld must be in [1, 64]", who, (long long)topk); return kErrArg; }
@@ -662,6 +756,10 @@ extern "C" int tl_moe_gate_up_swiglu(const void* x_bf16, const void* w13_packed,
     hipLaunchKernelGGL(moe_gate_up_lds_kernel, dim3(grid), dim3(kMoeWaves * 64), static_cast<size_t>(kLdsActBytes),
                        (hipStream_t)stream, (const uint16_t*)x_bf16, (const uint8_t*)w13_packed, s13, topk_idx,
                        (int)M, (int)topk, (int)expert_begin, (int)n_local, (int)D, (int)I, (uint16_t*)h_bf16);
+  } else if (gate_up_from_registers(M, n_local, D, I)) {
+    hipLaunchKernelGGL(moe_gate_up_kernel, dim3(grid), dim3(kMoeWaves * 64), 0, (hipStream_t)stream,
+                       (const uint16_t*)x_bf16, (const uint8_t*)w13_packed, s13, topk_idx, (int)M, (int)topk,
+                       (int)expert_begin, (int)n_local, (int)D, (int)I, (uint16_t*)h_bf16);
   } else {
     auto launch = [&](auto mq_tag) -> int {
       constexpr int MQ = decltype(mq_tag)::value, lds = kBigRing(MQ) + kBigRedGu;

@@ -25,6 +25,18 @@ struct ActOperand {
   v8bf v[4];
 };
 
+__device__ inline ActOperand load_act(const uint16_t* row_kblock, int g, bool live) {
+  ActOperand o;
+  const int off[4] = {16 * g, 16 * g + 8, 64 + 16 * g, 64 + 16 * g + 8};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    u32x4 d = {0u, 0u, 0u, 0u};
+    if (live) d = *reinterpret_cast<const u32x4*>(row_kblock + off[j]);
+    o.v[j] = __builtin_bit_cast(v8bf, d);
+  }
+  return o;
+}
+
 // acc[16 rows x 16 tokens] += dequant(W block) . x over one 128-wide K block: 4 chained
 // bf16 MFMAs on the block's bf16-rounded dequantised weights.
 __device__ inline v4f mfma_block_bf16(const v8i& w, float scale, const ActOperand& x, v4f acc) {
