@@ -723,6 +723,13 @@ static bool gate_up_from_registers(int64_t M, int64_t n_local, int64_t D, int64_
   return D <= 1024 || (D <= 2048 && (M < 14 || items <= 1 << 19)) || items <= 5 << 15;
 }
 
+// Down of 6 to 8 tokens: the LDS kernel takes h rows of up to 8 K blocks that fill the larger batches' two rounds of 4
+// waves a slot badly, as at up to 5 tokens.
+static bool down_from_lds(int64_t M, int64_t I) {
+  const int64_t KB = I / kBlock;
+  return M <= 5 || (M <= 8 && KB < 8 && (KB % 4 == 1 || KB % 4 == 2));
+}
+
 static int check_moe(const char* who, int64_t M, int64_t topk, int64_t n_local, int64_t D, int64_t I) {
   if (M < 1 || M > 16) { set_error("%s: M=%lld must be in [1, 16]", who, (long long)M); return kErrUnsupported; }
   if (topk < 1 || topk > 64) { set_error("%s: topk=%lld must be in [1, 64]", who, (long long)topk); return kErrArg; }
@@ -787,8 +794,10 @@ extern "C" int tl_moe_down_combine(const void* h_bf16, const void* w2_packed, co
   // Up to 5 tokens: h staged in LDS, sb hit experts per batch, two tiles' 16 waves on it; above, the
   // batches' staging and reductions cost more than streaming h beside the weights (D = 7168, I =
   // 2048, M = 4 / 5 / 6 / 8: 15.1 / 14.6 / 19.9 / 28.9 against 15.1 / 14.8 / 17.7 / 23.8 us;
-  // D = 6144, I = 1408: 10.9 / 11.1 / 14.6 / 21.3 against 11.7 / 11.7 / 13.9 / 18.6).
-  if (M <= 5 && h_bytes <= kDnHBytes && M * topk <= 64) {
+  // D = 6144, I = 1408: 10.9 / 11.1 / 14.6 / 21.3 against 11.7 / 11.7 / 13.9 / 18.6).  Where h has 1, 2, 5 or 6 K blocks,
+  // which the stream deals to 4 waves a slot, staging pays up to 8 tokens (D = 7168, M = 7 / 8: I = 128 7.2 / 7.9 against
+  // 7.9 / 8.7, I = 640 10.8 / 12.2 against 11.4 / 12.8; I = 512 10.1 / 11.3 against 9.4 / 10.3).
+  if (down_from_lds(M, I) && h_bytes <= kDnHBytes && M * topk <= 64) {
     // (the later batches are staged through registers: kStageChunks x 16 B per thread)
     const int64_t stage_cap = (D / 16) % 2 == 0 ? 2 * kLdsActBytes : kLdsActBytes;
     const int sb = static_cast<int>(std::min<int64_t>(kDnSlots, stage_cap / h_bytes));
