@@ -72,22 +72,13 @@ __device__ inline uint64_t lane_pairs_mask(int my_e, int n_local) {
   return wave_or_u64((my_e >= 0 && my_e < n_local) ? (1ull << my_e) : 0ull);
 }
 
-// Routing weight of (token r, local expert e); 0 when the token does not use it.  Pairs
-// beyond the 64 held by the lanes are read from memory.
-__device__ inline float routing_weight(const int32_t* __restrict__ topk_idx, const float* __restrict__ topk_w,
-                                       int my_e, float my_w, int pairs, int topk, int e0, int r, bool tok, int e) {
+// Routing weight of (token r, local expert e), from at most 64 lane-held pairs; 0 when the token does not use it.
+__device__ inline float routing_weight(int my_e, float my_w, int topk, int r, bool tok, int e) {
   float wj = 0.f;
   for (int k = 0; k < topk; ++k) {
-    const int src = r * topk + k;
-    int ee;
-    float v;
-    if (pairs <= 64) {
-      ee = __shfl(my_e, src & 63);
-      v = __shfl(my_w, src & 63);
-    } else {
-      ee = tok ? topk_idx[src] - e0 : -1;
-      v = tok ? topk_w[src] : 0.f;
-    }
+    const int src = (r * topk + k) & 63;
+    const int ee = __shfl(my_e, src);
+    const float v = __shfl(my_w, src);
     if (tok && ee == e) wj = v;
   }
   return wj;
@@ -101,7 +92,8 @@ constexpr int kLdsActBytes = 64 * 1024;  // activation staging limit (2 workgrou
 // Used when x [M, D] bf16 fits in 64 KB (M <= 4 at D = 7168).  The workgroup stages x in
 // LDS once; the waves then stream only weight fragments, kGuDepth blocks ahead through
 // ring_pipeline, and read their activation operands from LDS, so nothing but the weight
-// stream is waited on.  Work items, reduction and output as in moe_gate_up_kernel.
+// stream is waited on.  Work item = (slot, 16-channel tile); a persistent grid strides over n_hit * I/16 items, and
+// an item's partials are summed in wave order.
 __global__ __launch_bounds__(kMoeWaves * 64, 4) void moe_gate_up_lds_kernel(
     const uint16_t* __restrict__ x, const uint8_t* __restrict__ w13, const float* __restrict__ s13,
     const int32_t* __restrict__ topk_idx, int M, int topk, int e0, int n_local, int D, int I,
@@ -280,23 +272,23 @@ __global__ __launch_bounds__(kMoeWaves * 64, 4) void moe_gate_up_kernel(
 }
 
 // ------------------------------------------------------ down, LDS activations
-// Used when one hit expert's h rows [M, I] fit in 64 KB.  A workgroup covers TPW 16-row
-// output tiles with 8 waves each, so the staged h rows serve TPW tiles.  Hit experts are
-// taken `sb` at a time (sb * M * I * 2 <= 64 KB); the batch's h rows are staged in LDS and
+// For few tokens (down_from_lds) whose one hit expert's h rows [M, I] fit in kDnHBytes.  A workgroup covers two 16-row
+// output tiles (D % 128 == 0 makes their count even) with 8 waves each, so the staged h rows serve both.  Hit experts
+// are taken `sb` at a time (sb * M * I * 2 <= 128 KB); the batch's h rows are staged in LDS and
 // each tile's (slot, K block) items, dealt round-robin to its 8 waves, are streamed
 // kDnDepth ahead through ring_pipeline, one fp32 accumulator per slot.  After the stream
 // the same LDS holds the cross-wave partials: local wave j of a tile reduces slot j over
-// the tile's waves in order and rounds its weighted term to bf16 (the golden's per-term
-// rounding, as moe_down_kernel does); local wave 0 adds the terms in slot order.
-template <int TPW>
-__global__ __launch_bounds__(kDownWaves * 64 * TPW, 4) void moe_down_lds_kernel(
+// the tile's waves in order and rounds its weighted term to bf16, as the golden rounds each
+// term; local wave 0 adds the terms in slot order.
+constexpr int kDnTiles = 2;  // output tiles per workgroup
+__global__ __launch_bounds__(kDownWaves * 64 * kDnTiles, 4) void moe_down_lds_kernel(
     const uint16_t* __restrict__ h, const uint8_t* __restrict__ w2, const float* __restrict__ s2,
     const int32_t* __restrict__ topk_idx, const float* __restrict__ topk_w, int M, int topk, int e0,
     int n_local, int D, int I, int sb, uint16_t* __restrict__ y) {
   extern __shared__ __align__(16) uint8_t smem[];
   uint16_t* hl = reinterpret_cast<uint16_t*>(smem);  // [sb][M][I] during the stream
   v4f(*red)[kDnSlots][64] = reinterpret_cast<v4f(*)[kDnSlots][64]>(smem);  // after it
-  v4f(*term)[kDnSlots][64] = reinterpret_cast<v4f(*)[kDnSlots][64]>(smem + TPW * kDownRedBytes);
+  v4f(*term)[kDnSlots][64] = reinterpret_cast<v4f(*)[kDnSlots][64]>(smem + kDnTiles * kDownRedBytes);
   const int pairs = M * topk;
   const int my_e = lane_pair_expert(topk_idx, pairs, e0);
   const float my_w = lane_pair_weight(topk_w, pairs);
@@ -322,7 +314,7 @@ __global__ __launch_bounds__(kDownWaves * 64 * TPW, 4) void moe_down_lds_kernel(
   const int r = lane & 15, g = lane >> 4;
   const bool tok = r < M;
   const int row = min(r, M - 1);
-  const int rt = blockIdx.x * TPW + tt;
+  const int rt = blockIdx.x * kDnTiles + tt;
   v4f yacc = {0.f, 0.f, 0.f, 0.f};
 
   for (int s0 = 0; s0 < n_hit; s0 += sb) {
@@ -361,7 +353,7 @@ __global__ __launch_bounds__(kDownWaves * 64 * TPW, 4) void moe_down_lds_kernel(
         [&] {  // the batch's h rows into LDS while the first weight fetches are in flight
           if (s0 > 0) stage_commit(hl, stage_issue(h + static_cast<size_t>(s0) * M * I, h16), h16);
           if (wl < ns)
-            wj = routing_weight(topk_idx, topk_w, my_e, my_w, pairs, topk, e0, r, tok, nth_set_bit(mask, s0 + wl));
+            wj = routing_weight(my_e, my_w, topk, r, tok, nth_set_bit(mask, s0 + wl));
           if (s0 == 0) __builtin_amdgcn_s_waitcnt(0);  // this wave's part of the direct copy has landed
           __syncthreads();
         });
@@ -798,23 +790,14 @@ extern "C" int tl_moe_down_combine(const void* h_bf16, const void* w2_packed, co
   // which the stream deals to 4 waves a slot, staging pays up to 8 tokens (D = 7168, M = 7 / 8: I = 128 7.2 / 7.9 against
   // 7.9 / 8.7, I = 640 10.8 / 12.2 against 11.4 / 12.8; I = 512 10.1 / 11.3 against 9.4 / 10.3).
   if (down_from_lds(M, I) && h_bytes <= kDnHBytes && M * topk <= 64) {
-    // (the later batches are staged through registers: kStageChunks x 16 B per thread)
-    const int64_t stage_cap = (D / 16) % 2 == 0 ? 2 * kLdsActBytes : kLdsActBytes;
-    const int sb = static_cast<int>(std::min<int64_t>(kDnSlots, stage_cap / h_bytes));
-    // two output tiles per workgroup when the tile count is even: the staged h serves both
-    auto launch = [&](auto tpw_tag) -> int {
-      constexpr int TPW = decltype(tpw_tag)::value;
-      const size_t lds = std::max<size_t>(static_cast<size_t>(sb) * h_bytes, TPW * (kDownRedBytes + kDownTermBytes));
-      const void* fn = reinterpret_cast<const void*>(moe_down_lds_kernel<TPW>);
-      const int rc2 = allow_dynamic_lds(fn, static_cast<int>(lds), "moe_down_combine");
-      if (rc2) return rc2;
-      hipLaunchKernelGGL((moe_down_lds_kernel<TPW>), dim3(D / 16 / TPW), dim3(kDownWaves * 64 * TPW), lds,
-                         (hipStream_t)stream, (const uint16_t*)h_bf16, (const uint8_t*)w2_packed, s2, topk_idx, topk_w,
-                         (int)M, (int)topk, (int)expert_begin, (int)n_local, (int)D, (int)I, sb, (uint16_t*)y_bf16);
-      return 0;
-    };
-    rc = (D / 16) % 2 == 0 ? launch(std::integral_constant<int, 2>{}) : launch(std::integral_constant<int, 1>{});
+    // (the later batches are staged through registers: kStageChunks x 16 B per thread, 128 KB)
+    const int sb = static_cast<int>(std::min<int64_t>(kDnSlots, kDnHBytes / h_bytes));
+    const size_t lds = std::max<size_t>(static_cast<size_t>(sb) * h_bytes, kDnTiles * (kDownRedBytes + kDownTermBytes));
+    rc = allow_dynamic_lds(reinterpret_cast<const void*>(moe_down_lds_kernel), static_cast<int>(lds), "moe_down_combine");
     if (rc) return rc;
+    hipLaunchKernelGGL(moe_down_lds_kernel, dim3(D / 16 / kDnTiles), dim3(kDownWaves * 64 * kDnTiles), lds,
+                       (hipStream_t)stream, (const uint16_t*)h_bf16, (const uint8_t*)w2_packed, s2, topk_idx, topk_w,
+                       (int)M, (int)topk, (int)expert_begin, (int)n_local, (int)D, (int)I, sb, (uint16_t*)y_bf16);
   } else {
     auto launch = [&](auto mq_tag) -> int {
       constexpr int MQ = decltype(mq_tag)::value, lds = kBigRing(MQ) + kBigRedDn + kBigWeights;

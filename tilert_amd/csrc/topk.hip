@@ -533,11 +533,11 @@ __global__ __launch_bounds__(kTkThreads) void topk_kernel(const float* __restric
 // order, so the result is the chunked kernel's.
 template <int CPT>
 __global__ __launch_bounds__(kTkThreads) void topk_short_kernel(const float* __restrict__ logits, int64_t ld,
-                                                                int64_t valid_base, int k, int row0,
+                                                                int64_t valid_base, int k,
                                                                 int32_t* __restrict__ out) {
   __shared__ TopkShared sh;
   int slot = 0;
-  const int row = row0 + static_cast<int>(blockIdx.x);
+  const int row = static_cast<int>(blockIdx.x);
   const int n = row_valid(row, valid_base, ld);  // <= 1024 CPT (host)
   int32_t* o = out + static_cast<int64_t>(row) * k;
   if (n <= k) {  // every valid column, then -1 padding
@@ -621,7 +621,7 @@ extern "C" int tl_topk_rows(const float* logits, int64_t rows, int64_t ld, int64
     auto kern = longest <= 4 * kTkThreads ? topk_short_kernel<4>
                                           : (longest <= kShortCols ? topk_short_kernel<8> : topk_short_kernel<16>);
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(rows)), dim3(kTkThreads), 0, (hipStream_t)stream, logits, ld,
-                       valid_base, (int)k, 0, out);
+                       valid_base, (int)k, out);
     return check_launch("topk");
   }
   const TopkWs ws = carve(workspace, rows, p.chunks);
