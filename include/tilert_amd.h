@@ -128,8 +128,11 @@ int tl_fp8_gemm_packed(const void* a, const float* a_s, const void* b_packed, co
  * loops, harnesses that forbid hipMalloc): the same kernels and results (bit for bit), with
  * their scratch (split-K counters and partials, the activation image) in a static device
  * array of TL_FP8_GEMM_STATIC_SCRATCH_BYTES that each GPU holds until the process ends,
- * instead of a workspace argument.  The call allocates nothing; shapes whose scratch would
- * exceed the maximum fail with status 3 (every dense MLP shape of 7168 <-> 18432 up to
+ * instead of a workspace argument.  The call allocates nothing.  Which shapes it takes is fixed,
+ * whatever part of the array today's kernels use (19 MB beside an activation image at most): a shape
+ * counts an activation image (ceil(M/16) 16-row tiles of K bytes and their scales, for M <= 64) and fp32
+ * partials [M, N] of a K split (up to 4 for M <= 64), and fails with status 3 where these exceed
+ * the maximum, e.g. M = 64 at K = 655360 (every dense MLP shape of 7168 <-> 18432 up to
  * M = 256 fits).  Every call on a GPU shares that GPU's array: calls that overlap on one GPU
  * (different streams, or different threads without ordering) race; calls on one stream are
  * safe.  The array is zero when the library's code object loads and every call leaves its

@@ -57,8 +57,8 @@ def test_argument_errors_need_no_gpu():
     assert lib.tl_layernorm_rope_rotate(None, 4, None, None, 8, None, None, None, 1e-6, None) == 1
     assert b"null pointer" in lib.tl_last_error()
     assert lib.tl_layernorm_rope_rotate_ki(None, 0, None, None, 1, None, None, None, 1e-6, 5, None) == 1
-    assert lib.tl_fp8_gemm_workspace_bytes(32, 576, 7168) > 0  # narrow layer at M > 16: split K
-    # the allocation-free GEMM rejects a shape whose scratch exceeds its static array before
+    assert lib.tl_fp8_gemm_workspace_bytes(32, 576, 7168) > 0  # wide kernel: split K
+    # the allocation-free GEMM rejects a shape beyond the bound of those it takes before
     # touching the device (pointers are only checked for null and alignment)
     assert lib.tl_fp8_gemm_packed_static(256, 256, 256, 256, 256, 64, 16, 655360, None) == 3
     assert b"static maximum" in lib.tl_last_error()

@@ -61,7 +61,7 @@ GEMM_CASES = [
     # (M, N, K)
     (1, 256, 512),
     (4, 576, 7168),     # wkv_a: partial last scale row
-    (32, 576, 7168),    # 36 row tiles at M > 16: split-K in 4 slices
+    (32, 576, 7168),    # 36 row tiles, two 16-token tiles: wide kernel, split K
     (2, 7168, 6144),    # wide and long: 4 operand buffers per wave
     (4, 3072, 1536),    # wq_b
     (4, 4096, 512),     # wkv_b
@@ -71,29 +71,28 @@ GEMM_CASES = [
     (17, 512, 1024),
     (64, 1024, 2048),
     (256, 512, 1024),
-    (64, 2048, 7168),   # canonical: per-row-tile kernel, 4 token tiles, split-K; packed: wide kernel
-    (128, 2048, 7168),  # tiled kernel (M > 64) with split-K
+    (64, 2048, 7168),   # wide kernel (M > 32), split K
+    (128, 2048, 7168),  # wide kernel with 128-token groups (M > 64), split K
     (32, 1152, 2048),
-    (200, 400, 2048),   # 25 row tiles: a partly empty last 128-row group
+    (200, 400, 2048),   # 25 row tiles: a last tile group of one, a partly empty second token group
     (100, 7168, 1024),
-    # several row tiles per workgroup sharing each activation fragment
+    # GEMV (M = 16) with two row tiles per workgroup; wide kernel (M > 16) on wide, short layers
     (16, 7168, 1024),   # 2 row tiles, 1 token tile
     (16, 7168, 640),    # the same on the canonical (unpacked) layout
-    (32, 18432, 512),   # 4 row tiles, 2 token tiles
-    (24, 6144, 512),    # 2 row tiles, 2 token tiles
-    (48, 7168, 1024),   # 2 row tiles, 4 token tiles
-    (64, 12288, 512),   # 4 row tiles, 4 token tiles
-    # M > 32 (or > 16 with K split in <= 2), packed: wide MFMA GEMM (F row tiles per
-    # workgroup, S K ranges)
-    (65, 128, 512),     # F = 4: 2 slices, each split over all 4 K blocks: 4 partials
-    (192, 1024, 2048),  # F = 8: 2 token groups, the second half full; 8 tiles x 16 K ranges
-    (40, 2048, 1024),   # one token group with 3 of its 8 fragments past M
-    (200, 640, 2048),   # F = 5
-    (200, 768, 2048),   # F = 6
-    (200, 1152, 2048),  # F = 9
-    (200, 4352, 1024),  # F = 8, K ranges of 3, 3 and 2 blocks
+    (32, 18432, 512),   # K of 4 blocks
+    (24, 6144, 512),
+    (48, 7168, 1024),
+    (64, 12288, 512),
+    # wide MFMA GEMM (its row-tile counts and K splits: test_gpu_wide_plans.py)
+    (65, 128, 512),     # 8 row tiles, unsplit
+    (192, 1024, 2048),  # 2 token groups, the second half full
+    (40, 2048, 1024),   # one token group with its last fragment past M
+    (200, 640, 2048),   # 40, 48 and 72 row tiles
+    (200, 768, 2048),
+    (200, 1152, 2048),
+    (200, 4352, 1024),  # 272 row tiles, two token groups
     (255, 2048, 1024),  # last token fragment 15/16 full, second token group
-    (33, 7168, 512),    # 3 of 8 token fragments valid, 4 K ranges of one block
+    (33, 7168, 512),    # 3 of 4 token fragments valid
 ]
 
 
@@ -112,9 +111,9 @@ def test_fp8_gemm_vs_oracle(cuda, M, N, Kd):
     if Kd % 512 == 0:
         packed = K.pack_weight(wq.to(cuda), ws.to(cuda))
         outp = K.fp8_gemm(xq.to(cuda), xs.to(cuda), packed)
-        if M <= 16 or N % 128:  # the same GEMV kernel on both layouts
+        if M <= 16 or N % 128:
             assert torch.equal(outp, out), "packed-weight GEMM differs from the canonical one"
-        else:  # the wide MFMA GEMM (packed) and the GEMV / tiled kernel (canonical) sum differently
+        else:  # (the layouts' equality here: test_gpu_wide_edges.py, test_gpu_wide_plans.py)
             assert torch.equal(outp, K.fp8_gemm(xq.to(cuda), xs.to(cuda), packed)), "not deterministic"
             assert_gemm_close(outp, ref.fp8_gemm(xq, xs, wq, ws), f"packed M={M} N={N} K={Kd}")
 
@@ -183,5 +182,5 @@ def test_fp8_gemm_split_k_repeatable(cuda, M, N, Kd):
     torch.cuda.synchronize()
     for o in outs:
         assert torch.equal(o, first)
-    for o in outs_c:  # packed M > 16 with N % 128 = 0 may run the wide kernel; canonical: another one
+    for o in outs_c:
         assert torch.equal(o, first if (M <= 16 or N % 128) else first_c)

@@ -1,7 +1,7 @@
 """The allocation-free entry point ``tl_fp8_gemm_packed_static`` (scratch in a static device
 array) against ``tl_fp8_gemm_packed`` with a caller workspace, through the C ABI: bit-identical
 on two calls in a row (the second smaller, so it runs over the first call's leftover scratch),
-and a clear error for a shape whose scratch exceeds the static maximum."""
+and a clear error for a shape beyond the bound of those it takes."""
 import pytest
 import torch
 
@@ -43,11 +43,11 @@ def _static(xq, xs, packed, M, N, Kd, dev):
 
 
 @pytest.mark.parametrize("first,second", [
-    # the wide MFMA GEMM with a K split (fp32 partials), then the split-K GEMV over its leftovers
+    # the wide MFMA GEMM with a K split (fp32 partials), then a narrow layer's over its leftovers
     ((256, 7168, 4096), (40, 576, 7168)),
-    # GEMV with the activation image and 4 row tiles, then a plain M = 4 GEMV (no scratch)
+    # the wide MFMA GEMM at 64 tokens, then a plain M = 4 GEMV (no scratch)
     ((64, 18432, 7168), (4, 1024, 2048)),
-    # split-K GEMV at M > 16, then a smaller split-K GEMV: the counters must be zero again
+    # split K, then a smaller layer with split K: the counters must be zero again
     ((48, 1024, 7168), (17, 512, 2048)),
     # the largest dense-MLP shapes of the M sweep (down 18432 -> 7168 at M = 256 has the
     # largest scratch of the sweep), then up at M = 64
@@ -68,7 +68,8 @@ def test_static_matches_workspace_entry_point(cuda, first, second):
 def test_static_rejects_shapes_beyond_the_maximum(cuda):
     lib = _lib.load()
     dev = cuda
-    # M = 64 over K = 655360: the GEMV's activation image (64 x K bytes + scales) exceeds 40 MiB
+    # M = 64 over K = 655360: the fixed bound of the shapes it takes counts an activation image there (64 x K bytes +
+    # scales), which exceeds 40 MiB
     M, N, Kd = 64, 16, 655360
     a = torch.zeros(M, Kd, dtype=torch.float8_e4m3fn, device=dev)
     a_s = torch.ones(M, Kd // 128, device=dev)

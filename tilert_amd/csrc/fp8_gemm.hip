@@ -636,7 +636,7 @@ __global__ __launch_bounds__(kWideWaves * 64) void fp8_gemm_wide_kernel(
 // rate is 0.02).  Fitted to every (F, S) at nine layer shapes and M = 24..256:
 //   * K blocks: (2 F + 8 TJ + 1) copies each, times the blocks of a range and the rounds of
 //     256 workgroups;
-//   * never less than the weight itself at 5.5 TB/s (7168 <-> 18432: 937 units);
+//   * never less than the weight itself at 5.5 TB/s (7168 <-> 18432: 934 units);
 //   * a split: publishing and the counter (1.5 us; 3 us with 128-token tiles), and per range one dependent
 //     round trip of its slot (4 F TJ KB) in the last workgroup's sum.
 // Narrow layers take small tiles and few ranges (7168 -> 1536 at M = 64: F = 4, S = 6..8
@@ -753,7 +753,7 @@ template <bool PACKED>
 static int launch_gemm(const uint8_t* A, const float* As, const uint8_t* B, const float* Bs,
                        const OutRoute& out, int M, int N, int K, void* workspace, hipStream_t st) {
   const GemmPlan p = plan_gemm(M, N, K);
-  // From M = 16 on the activations are first rearranged into the workspace (act_image_kernel).
+  // For the GEMV, from M = 16 on, the activations are first rearranged into the workspace (act_image_kernel).
   const uint8_t* xa = A;
   const float* xsa = As;
   if (p.xf) {
@@ -1110,7 +1110,8 @@ int scratch_for_current_device(void** out) {
 }  // namespace
 
 // Which shapes the static entry point takes is part of its interface, so it follows a fixed
-// bound and not the plans: the scratch of a K-split GEMV (M <= 64: the activation image
+// bound and not the plans, so that no change of a plan takes a shape away or lets callers rely on one that the next plan
+// refuses: the scratch of a K-split GEMV (M <= 64: the activation image
 // and the partials) or of a split 128-row-tile GEMM (M > 64) where N % 128 != 0 or, at M =
 // 17..32, a balanced round of 256 workgroups of 4..9 row tiles would split K more than 4 ways.
 // The plans need at most 19 MB beside the image.
@@ -1149,7 +1150,7 @@ extern "C" int tl_fp8_gemm_packed_static(const void* a, const float* a_s, const 
   if (rc) return rc;
   const size_t need = std::max(plan_workspace_bytes(M, N, K), static_bound_bytes(M, N, K));
   if (need > TL_FP8_GEMM_STATIC_SCRATCH_BYTES) {
-    set_error("%s: M=%lld N=%lld K=%lld needs %zu bytes of scratch, above the static maximum of %zu", who,
+    set_error("%s: M=%lld N=%lld K=%lld counts %zu bytes of scratch, above the static maximum of %zu", who,
               (long long)M, (long long)N, (long long)K, need, static_cast<size_t>(TL_FP8_GEMM_STATIC_SCRATCH_BYTES));
     return kErrUnsupported;
   }
