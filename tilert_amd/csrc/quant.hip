@@ -297,17 +297,24 @@ __device__ inline float norm_factor(const float (&part)[kNormVirt / 64], int dim
   return 1.0f / __builtin_sqrtf(tot / static_cast<float>(dim) + eps);
 }
 
-// Outputs (y and its codes) that the whole-row kernel stores non-temporally: between 3 and 40 MB, about what the L2s
-// hold and would write back at the kernel's end.  Smaller ones the next kernel reads from L2, and of larger ones it
-// finds in the Infinity Cache what non-temporal stores leave to memory.  us, norm + a kernel that reads the codes / that
-// reads y, non-temporal against temporal: 256 x 1536 5.4 / 5.5 against 5.2 / 5.4; 2048 x 1536 9.4 / 11.0 against
-// 10.1 / 12.2; 8192 x 1536 23.9 / 28.5 against 24.9 / 29.1; 256 x 7168 8.0 / 8.7 against 8.1 / 9.1; 1024 x 7168
-// 13.6 / 16.6 against 14.8 / 17.9; 2048 x 7168 24.0 / 30.6 against 25.0 / 29.1; 4096 x 7168 45.2 / 53.8 against
-// 43.3 / 50.9 (with 16 FP8 GEMMs 7168 -> 576 on its codes 272 against 263), though its norm alone takes 28.3 against 33.1.
+// Which outputs the whole-row kernel stores non-temporally: from 3 MB of them (y and codes) both, about what the L2s
+// hold and would write back at the kernel's end; smaller ones the next kernel reads from L2.  From 40 MB only y, and only
+// where codes are given: what is stored non-temporally then goes to memory, where plain stores leave it in the Infinity
+// Cache, and the codes are what the next GEMMs read.  us, norm + a kernel that reads the codes / that reads y,
+// non-temporal against plain: 256 x 1536 5.4 / 5.5 against 5.2 / 5.4; 2048 x 1536 9.4 / 11.0 against 10.1 / 12.2;
+// 8192 x 1536 23.9 / 28.5 against 24.9 / 29.1; 256 x 7168 8.0 / 8.7 against 8.1 / 9.1; 1024 x 7168 13.6 / 16.6 against
+// 14.8 / 17.9; 2048 x 7168 24.0 / 30.6 against 25.0 / 29.1; 4096 x 7168 45.2 / 53.8 against 43.3 / 50.9.  4096 x 7168 with
+// the index keys behind it, both / y only / plain: 32.1 / 33.0 / 35.8; with 16 FP8 GEMMs 7168 -> 2112 on its codes too
+// 334.8 / 327.1 / 327.7; where y is read as well 355 / 348 / 347.
+enum NormNt { kNtNone, kNtY, kNtBoth };
 constexpr int64_t kNormNtMin = 3 << 20, kNormNtMax = 40 << 20;
+__host__ inline NormNt norm_nt(int64_t rows, int64_t dim, bool codes) {
+  const int64_t bytes = rows * dim * (codes ? 3 : 2);
+  return bytes < kNormNtMin ? kNtNone : (bytes < kNormNtMax ? kNtBoth : (codes ? kNtY : kNtNone));
+}
 
 // Normalise (and quantise) chunk c of a row: 16 consecutive lanes hold a 128-element group.
-template <bool NT>
+template <NormNt NT>
 __device__ inline void norm_chunk(const uint4& raw, const float (&gv)[8], float r, bool live, int c, int row, int dim,
                                   uint16_t* __restrict__ y, uint8_t* __restrict__ y8, float* __restrict__ ys,
                                   int scale_mode) {
@@ -321,7 +328,7 @@ __device__ inline void norm_chunk(const uint4& raw, const float (&gv)[8], float 
     q[2 * j] = bf16_to_f32(b[j] & 0xffff);
     q[2 * j + 1] = bf16_to_f32(b[j] >> 16);
   }
-  if (live) store_chunk<NT>(reinterpret_cast<u32x4n*>(y + static_cast<int64_t>(row) * dim) + c, u32x4n{b[0], b[1], b[2], b[3]});
+  if (live) store_chunk<NT != kNtNone>(reinterpret_cast<u32x4n*>(y + static_cast<int64_t>(row) * dim) + c, u32x4n{b[0], b[1], b[2], b[3]});
   if (!y8) return;  // kernel-uniform
   float amax = 0.f;
 #pragma unroll
@@ -330,7 +337,7 @@ __device__ inline void norm_chunk(const uint4& raw, const float (&gv)[8], float 
   const float sc = group_scale(amax, scale_mode);
   const uint2 code = quant8_e4m3(q, sc);
   if (live) {
-    store_chunk<NT>(reinterpret_cast<u32x2n*>(y8 + static_cast<int64_t>(row) * dim) + c, u32x2n{code.x, code.y});
+    store_chunk<NT == kNtBoth>(reinterpret_cast<u32x2n*>(y8 + static_cast<int64_t>(row) * dim) + c, u32x2n{code.x, code.y});
     if ((c & 15) == 0) ys[static_cast<int64_t>(row) * (dim / kBlock) + (c >> 4)] = sc;
   }
 }
@@ -367,7 +374,7 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_quant_kernel(
   __syncthreads();
   const float r = norm_factor(part, dim, eps);
   const float gv[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-  norm_chunk<false>(mine, gv, r, live, c, row, dim, y, y8, ys, scale_mode);
+  norm_chunk<kNtNone>(mine, gv, r, live, c, row, dim, y, y8, ys, scale_mode);
 }
 
 // Many rows (norm_rows_min): HBM-bound.  One workgroup takes whole rows, kept in registers between the sum and the outputs (the slices above read
@@ -379,7 +386,7 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_quant_kernel(
 // request of a next one repeats the last row for nothing.
 // Instances for 1, 2, 4, 5, 6 and 8 chunks a thread: registers go with the chunks (5: 158 VGPRs, three workgroups per CU;
 // 10240 wide rows in the instance for 8 chunks, with one, 1024 / 4096 rows 23.5 / 76 us, in their own 11.7 / 39.3).
-template <int NC, bool NT>  // chunks per thread: dim <= 2048 NC
+template <int NC, NormNt NT>  // chunks per thread: dim <= 2048 NC
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_quant_rows_kernel(
     const uint16_t* __restrict__ x, const float* __restrict__ gamma, float eps, int rows, int dim,
     uint16_t* __restrict__ y, uint8_t* __restrict__ y8, float* __restrict__ ys, int scale_mode) {
@@ -465,11 +472,12 @@ extern "C" int tl_rmsnorm_quant(const void* x_bf16, const float* gamma, float ep
     else slice(std::integral_constant<int, 2>{});
     return check_launch("rmsnorm_quant");
   }
-  const int64_t out_bytes = rows * dim * (y_fp8 ? 3 : 2);
-  const bool nt = out_bytes >= kNormNtMin && out_bytes < kNormNtMax;
+  const NormNt nt = norm_nt(rows, dim, y_fp8 != nullptr);
   auto launch = [&](auto nc) {
     constexpr int NC = decltype(nc)::value;
-    hipLaunchKernelGGL((nt ? rmsnorm_quant_rows_kernel<NC, true> : rmsnorm_quant_rows_kernel<NC, false>),
+    const auto kern = nt == kNtNone ? rmsnorm_quant_rows_kernel<NC, kNtNone>
+                                    : (nt == kNtY ? rmsnorm_quant_rows_kernel<NC, kNtY> : rmsnorm_quant_rows_kernel<NC, kNtBoth>);
+    hipLaunchKernelGGL(kern,
                        dim3(static_cast<unsigned>(rows < kNormRowsGrid ? rows : kNormRowsGrid)), dim3(kNormThreads), 0,
                        (hipStream_t)stream, (const uint16_t*)x_bf16, gamma, eps, (int)rows, (int)dim, (uint16_t*)y_bf16,
                        (uint8_t*)y_fp8, y_scale, scale_mode);
